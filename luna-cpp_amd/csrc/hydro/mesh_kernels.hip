@@ -2,43 +2,33 @@
 // and the update, one per face for the fluxes. FP64, -ffp-contract=off; each cell sums over its face list in list order,
 // so every run gives the same bits, and those of the CPU restatement of the reference's arithmetic.
 //
-// Memory (kernels.hpp): a neighbour is one 128 B cell row (position, centroid, state) and a face one 64 B record; the
-// lists are stored in 64-cell slices, so a wavefront reads the t-th entries of its cells as one contiguous run and the
-// entries of the next group are in flight while the current group is summed; work-groups are mapped so that each XCD
-// takes a contiguous run of cells (neighbours in Morton order share its L2).
+// Memory (kernels.hpp): a neighbour is one 128 B cell row (position, centroid, state); the lists are stored in 64-cell
+// slices, so a wavefront reads the t-th entries of its cells as one contiguous run; the rows an entry names go through LDS
+// in whole lines, two entries ahead of the sums (Stage); work-groups are mapped so that each XCD takes a contiguous run of
+// cells (neighbours in Morton order share its L2).
 #include <hip/hip_fp16.h>
 
 #include <type_traits>
 
+#include "exact_math.hpp"
 #include "kernels.hpp"
 
-// Tuning knobs (compile-time; the defaults are the measured best): entries of the sweep's first walk and of its limiter
-// walk loaded together, flux rows of the update loaded together, and the occupancy floor (waves per SIMD) of the sweep,
-// flux and LaneSweep kernels.
-#ifndef LUNA_SWEEP_UNROLL
-#define LUNA_SWEEP_UNROLL 1
-#endif
+// Tuning knobs (compile-time; the defaults are the measured best): entries of the sweep's limiter walk loaded together, flux
+// rows of the update loaded together, and the occupancy floor (waves per SIMD) of the sweep, flux and LaneSweep kernels.
 #ifndef LUNA_LIMIT_UNROLL
 #define LUNA_LIMIT_UNROLL 4
 #endif
 #ifndef LUNA_UPDATE_UNROLL
 #define LUNA_UPDATE_UNROLL 4
 #endif
-#ifndef LUNA_SWEEP_WAVES
-#define LUNA_SWEEP_WAVES 3
+#ifndef LUNA_SWEEP_WAVES  // 2 (178 and 188 VGPRs, no spill): 0.72 ms static and 0.44 ms moving; 3 spills 32 to 120 B: 0.74 and 0.74
+#define LUNA_SWEEP_WAVES 2
 #endif
 #ifndef LUNA_FLUX_WAVES
 #define LUNA_FLUX_WAVES 1
 #endif
 #ifndef LUNA_LANE_WAVES  // LaneSweep's occupancy floor: 2 and 8 lanes measured best at 2 waves (no spill), 4 lanes at 3
 #define LUNA_LANE_WAVES(L) ((L) == 4 ? 3 : 2)
-#endif
-// 1: every sweep takes the neighbours' range (min, max of W) in a loop of its own after the fit, re-reading the
-// neighbours' W (cache-resident), instead of carrying it through the first walk (20 registers fewer there); 0: only the
-// moving FP64 sweep does (the static one fits 3 waves per SIMD without it; the moving one spills with it carried). The
-// reduced-precision sweeps load two entries together and carry the range (their float sums are half the registers).
-#ifndef LUNA_RANGE_PASS
-#define LUNA_RANGE_PASS 0
 #endif
 
 namespace luna {
@@ -147,6 +137,84 @@ __device__ __forceinline__ void load_near(const Geo& g, int slot, int j, Near<D>
     n.cs = row[C::CS];
 }
 
+// A wavefront's neighbour rows through LDS. A lane that loads its own neighbour's row itself touches a 128 B line per 16 B
+// load, and a CU's L1 looks up one line a cycle: the rows of 64 neighbours cost 7 x 64 lookups, which bound the list walk
+// (5.6 thousand cycles an entry at 12 wavefronts a CU). Here the 16 B chunks of all 64 rows are dealt to the lanes in order
+// (chunk q to lane q mod 64 of load q / 64, of row q / CHUNKS), so that a load covers whole rows, and go to LDS without
+// passing through registers, back to back (a row at 16 CHUNKS bytes times its lane). Chunks with neither x, c, W nor c_s
+// (V and r) are skipped. Two buffers: one is read while the other is in flight.
+typedef __attribute__((address_space(3))) double lds_double;
+typedef double double2v __attribute__((ext_vector_type(2)));
+template <int D>
+struct Stage {
+    static constexpr int CHUNKS = D == 3 ? 6 : 5, ROW = 2 * CHUNKS;  // a staged row: [x, c, W, c_s]
+    static constexpr int DOUBLES = 2 * 64 * ROW;                      // both buffers
+    static constexpr int SKIP = D;                                    // staged chunks before it are a row's first, the others its from GEO_ROW / 2 on
+    static constexpr int PERIOD = D == 3 ? 3 : 5;                     // load k + PERIOD takes the same chunks of rows 32 further (3D)
+    int from[PERIOD], chunk[PERIOD];  // per load: 4 x the lane whose neighbour this lane fetches for, the chunk of its row
+    unsigned at[CHUNKS];              // per load: the next fetch's source, in chunks from the first cell row
+    lds_double* buffer;
+    unsigned row;  // the LDS address of this lane's row in buffer 0
+
+    __device__ __forceinline__ void init(int lane, lds_double* lds) {
+#pragma unroll
+        for (int k = 0; k < PERIOD; ++k) {
+            const int q = k * 64 + lane, c = q % CHUNKS;
+            from[k] = q / CHUNKS * 4;
+            chunk[k] = c < SKIP ? c : c - SKIP + GEO_ROW / 2;
+        }
+        buffer = lds;
+        row = (unsigned)(size_t)lds + lane * ROW * 8;
+    }
+    // The sources of a fetch of the cells j's rows (one a lane; every lane active).
+    __device__ __forceinline__ void address(int j) {
+#pragma unroll
+        for (int k = 0; k < CHUNKS; ++k)
+            at[k] = (unsigned)__builtin_amdgcn_ds_bpermute(from[k % PERIOD] + k / PERIOD * 128, j) << 3 | (unsigned)chunk[k % PERIOD];
+    }
+    __device__ __forceinline__ void fetch(const double* cell, int b) const {
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int k = 0; k < CHUNKS; ++k) {
+            const char* src = reinterpret_cast<const char*>(cell) + (size_t)at[k] * 16;
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                             (__attribute__((address_space(3))) void*)(buffer + b * (64 * ROW) + k * 128), 16, 0, 0);
+        }
+        asm volatile("" ::: "memory");
+    }
+    // This lane's row in buffer b, whose fetch may be followed by one other of CHUNKS loads that is still in flight. The reads
+    // are complete when this returns, so that the next fetch may overwrite the buffer.
+    __device__ __forceinline__ void read(int b, Near<D>& n) const {
+        const unsigned p = row + b * (64 * ROW * 8);
+        double2v d[CHUNKS];
+        if constexpr (D == 3)
+            asm volatile(
+                "s_waitcnt vmcnt(6)\n\tds_read_b128 %0, %6\n\tds_read_b128 %1, %6 offset:16\n\tds_read_b128 %2, %6 offset:32\n\t"
+                "ds_read_b128 %3, %6 offset:48\n\tds_read_b128 %4, %6 offset:64\n\tds_read_b128 %5, %6 offset:80\n\ts_waitcnt lgkmcnt(0)"
+                : "=&v"(d[0]), "=&v"(d[1]), "=&v"(d[2]), "=&v"(d[3]), "=&v"(d[4]), "=&v"(d[CHUNKS - 1])
+                : "v"(p)
+                : "memory");
+        else
+            asm volatile(
+                "s_waitcnt vmcnt(5)\n\tds_read_b128 %0, %5\n\tds_read_b128 %1, %5 offset:16\n\tds_read_b128 %2, %5 offset:32\n\t"
+                "ds_read_b128 %3, %5 offset:48\n\tds_read_b128 %4, %5 offset:64\n\ts_waitcnt lgkmcnt(0)"
+                : "=&v"(d[0]), "=&v"(d[1]), "=&v"(d[2]), "=&v"(d[3]), "=&v"(d[4])
+                : "v"(p)
+                : "memory");
+        const auto v = [&](int k) { return k & 1 ? d[k / 2].y : d[k / 2].x; };
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            n.x[a] = v(a);
+            n.c[a] = v(D + a);
+        }
+#pragma unroll
+        for (int w = 0; w < D + 2; ++w) n.W[w] = v(2 * D + w);
+        n.cs = v(3 * D + 2);
+    }
+    // Nothing in flight to LDS any more.
+    __device__ __forceinline__ void drain() const { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+};
+
 // The gradient rows of the precision policies (precision.hpp:26-54, 55-130). FP16 (grad16): each group (rho, v, P) of the
 // cell's gradient is scaled by 2^k so that its largest component is in [2^14, 2^15) (k = 0 for an all-zero group, within
 // [-114, 126]); the three k are kept as int8 in one 32-bit word per cell. The conversions are the hardware's
@@ -227,37 +295,94 @@ __device__ __forceinline__ constexpr G finite_max() {
     return sizeof(G) == 8 ? (G)1.7976931348623157e308 : (G)3.4028234663852886e38f;
 }
 
+// Division and square root of the sweep: the general operators, or (Fast) the correctly rounded ones of exact_math.hpp, whose
+// operands the caller checks.
+template <bool Fast>
+struct Arith {
+    static __device__ __forceinline__ Divisor by(double b) {
+        if constexpr (Fast) return divisor(b);
+        return Divisor{b, 0.0};
+    }
+    static __device__ __forceinline__ double quotient(double a, const Divisor& d) {
+        if constexpr (Fast) return over(a, d);
+        return a / d.b;
+    }
+    static __device__ __forceinline__ double square_root(double x) {
+        if constexpr (Fast) return root(x);
+        return sqrt(x);
+    }
+};
+
+// fmin and fmax of values that arithmetic made (the instruction alone: fmin() first quiets operands that came from memory).
+__device__ __forceinline__ double lower(double a, double b) {
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ double higher(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float lower(float a, float b) { return fminf(a, b); }
+__device__ __forceinline__ float higher(float a, float b) { return fmaxf(a, b); }
+
 // The sweep's per-cell sums (finite_volume.hpp:486-515), in list order. G: the fit's type (double, or float for the
-// reduced-precision policies, whose range is of W_j - W_i, rounded once, :466-469, 510-512).
-template <int D, bool Moving, bool Grad, int Rule, class G = double, bool RangePass = false>
+// reduced-precision policies, whose range is of W_j - W_i, rounded once, :466-469, 510-512). Fast: ok tells whether every
+// operand was in the range of the fast operators.
+template <int D, bool Moving, bool Grad, int Rule, class G = double, bool Fast = false>
 struct Sums {
     static constexpr int V = D + 2, U = D + 1;
     static constexpr bool exact = sizeof(G) == 8;
-    double surface = 0, smallest_face = INFINITY, max_angle = 0, smallest = INFINITY;
+    using Op = Arith<Fast>;
+    double max_angle = 0, smallest = INFINITY;
     G lo[V], hi[V], M[U][U], b[V][U];
+    bool ok = true;
 
-    __device__ __forceinline__ void init() {
+    __device__ __forceinline__ void init_range() {
 #pragma unroll
         for (int v = 0; v < V; ++v) {
             lo[v] = finite_max<G>();
             hi[v] = -finite_max<G>();
+        }
+    }
+    __device__ __forceinline__ void init() {
+        init_range();
+#pragma unroll
+        for (int v = 0; v < V; ++v)
 #pragma unroll
             for (int p = 0; p < U; ++p) b[v][p] = 0;
-        }
 #pragma unroll
         for (int p = 0; p < U; ++p)
 #pragma unroll
             for (int s = 0; s < U; ++s) M[p][s] = 0;
     }
+    // neighbour_range (:572-588): the range of the neighbours' W; faces under 1e-6 of the surface are left out by the caller.
+    __device__ __forceinline__ void range(const double* Wn, const double* Wi) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            const G value = exact ? (G)Wn[v] : (G)(Wn[v] - Wi[v]);
+            lo[v] = lower(lo[v], value);
+            hi[v] = higher(hi[v], value);
+        }
+    }
     __device__ __forceinline__ void add(const Geo& g, const Near<D>& n, const double* xi, const double* centroid, const double* Wi,
-                                        double csi, double ri, double courant) {
+                                        double csi, double ri, double courant, double tiny) {
         double d[D];
         separation<D>(g, xi, n.x, d);
         const double magnitude = n.mag;
-        surface += magnitude;
-        smallest_face = fmin(smallest_face, magnitude);
-        const double dist = sqrt(dot<D>(d, d));
-        if constexpr (Moving) max_angle = fmax(max_angle, face_angle<D>(magnitude) / (0.5 * dist));
+        const double dd = dot<D>(d, d), dist = Op::square_root(dd);
+        const Divisor by_dist = Op::by(dist);
+        if constexpr (Fast) ok = ok && plain(dd);
+        if constexpr (Moving) {
+            if constexpr (Fast && D == 3) {  // face_angle<3>: 1 / pi rounded to nearest, as divisor() would give it
+                ok = ok && plain(magnitude);
+                const double angle = root(over(magnitude, Divisor{M_PI, M_1_PI}));
+                max_angle = higher(max_angle, over(angle, Divisor{0.5 * dist, 2.0 * by_dist.y}));
+            } else {
+                max_angle = fmax(max_angle, Op::quotient(face_angle<D>(magnitude), Divisor{0.5 * dist, 2.0 * by_dist.y}));
+            }
+        }
         if constexpr (Grad) {
             G X[U];
             X[0] = 1;
@@ -273,19 +398,17 @@ struct Sums {
                 const double dW = n.W[v] - Wi[v];
 #pragma unroll
                 for (int p = 0; p < U; ++p) b[v][p] += w * X[p] * (G)dW;
-                if constexpr (!RangePass) {
-                    const G value = exact ? (G)n.W[v] : (G)dW;
-                    lo[v] = fmin(lo[v], value);
-                    hi[v] = fmax(hi[v], value);
-                }
             }
+            if (!(magnitude < tiny)) range(n.W, Wi);
         }
         if constexpr (Rule == 0) {  // FaceStep (:1079-1089) from this side
             double dv[D];
 #pragma unroll
             for (int a = 0; a < D; ++a) dv[a] = n.W[1 + a] - Wi[1 + a];
-            const double vsig = csi + n.cs - dot<D>(dv, d) / dist;
-            if (vsig > 0) smallest = fmin(smallest, courant * ((dist + ri) / vsig));
+            const double vsig = csi + n.cs - Op::quotient(dot<D>(dv, d), by_dist);
+            if constexpr (Fast) ok = ok && plain(vsig);
+            const double term = courant * Op::quotient(dist + ri, Op::by(vsig));
+            smallest = vsig > 0 && term < smallest ? term : smallest;
         }
     }
 };
@@ -293,247 +416,297 @@ struct Sums {
 // The sweep (finite_volume.hpp:463-569 Sweep::operator(), double policy) with the time step's terms (:1040-1104) fused:
 // each cell takes its own term and, for every face of its list, the face term with its own radius. The pair term vsig and
 // |d| have the same bits from either side, so the minimum is the reference's (the face kernel's terms are the same set).
-// The first block also resets the other dt slot and the step's fallback counters. Limit: 0 none, 1 the face-centroid
-// limiter, 2 the same limiter recording the learned limiter's features and troubled-cell flag (the gradients are those of 1).
-template <int D, bool Moving, bool Grad, int Limit, int Rule, int Prec = 0>
-__global__ __launch_bounds__(CELL_BLOCK, Limit == 2 ? 1 : LUNA_SWEEP_WAVES) void k_sweep(Geo g, Rows r, Gas gas, double courant, Counters c) {
+// Limit: 0 none, 1 the face-centroid limiter, 2 the same limiter recording the learned limiter's features and troubled-cell
+// flag (the gradients are those of 1).
+// What bounds it: at two wavefronts a SIMD the list walk takes two thirds of a wavefront's time (175 VALU instructions and 6
+// row loads an entry) and the limiter a third. Measured at 128^3 (waves in every variable and a blast), static: 0.95 ms with
+// rows loaded lane by lane, the compiler's divisions, the range walked again for tiny faces and the clips in branches; 0.79
+// with the surface summed first, the fast operators and the clips side by side; 0.72 with the rows through LDS. Moving, 104^3:
+// 0.63, 0.62, 0.44 ms. One wavefront, a slice of 64 cells; Fast as Arith: returns false, having written
+// nothing, if some operand of the wavefront was out of the fast operators' range. smallest: the smallest time-step term.
+template <int D, bool Moving, bool Grad, int Limit, int Rule, int Prec, bool Fast>
+__device__ __forceinline__ bool sweep_slice(const Geo& g, const Rows& r, double courant, int block, lds_double* lds, double& smallest) {
     constexpr int V = D + 2, U = D + 1;
     using G = typename std::conditional<Prec == 0, double, float>::type;
     constexpr bool exact = Prec == 0;
     static_assert(exact || Limit < 2, "the learned limiter's features need the double policy");
     using C = CellAt<D>;
-    const int i = xcd_block() * CELL_BLOCK + threadIdx.x;
+    using Op = Arith<Fast && exact>;
+    const unsigned lane = threadIdx.x;
+    const int i = block * CELL_BLOCK + (int)lane;
+    const bool here = i < g.N;
+    const double* mine = g.cell + (size_t)(here ? i : g.N - 1) * CELL_ROW;
+    double Wi[V], xi[D], centroid[D];
+#pragma unroll
+    for (int v = 0; v < V; ++v) Wi[v] = mine[C::W + v];
+    const double ci = mine[C::CS], ri = mine[C::RAD];
+    load_vec<D>(mine + C::X, xi);
+    load_vec<D>(mine + C::C, centroid);
+    Sums<D, Moving, Grad, Rule, G, Fast> s;
+    s.init();
+    const int first = g.slice[block];
+    const int* other = g.other + first;       // the slice's entries: entry t of lane l at t SLICE + l
+    const double* geometry = g.slot + first;  // |A|; the face offsets a + 1 times g.slots further
+    const int depth = ((block + 1 < (g.N + SLICE - 1) / SLICE ? g.slice[block + 1] : (int)g.slots) - first) / SLICE;
+    const int count = here ? g.count[i] : 0;
+    double tiny = 0;
+    if constexpr (Grad) {  // the surface first: which faces the range leaves out (walking the list again for them cost 0.15 ms at 128^3)
+        double surface = 0;
+        constexpr int US = 8;
+        for (int t = 0; t < depth; t += US) {
+            double m[US];
+#pragma unroll
+            for (int u = 0; u < US; ++u) m[u] = (geometry + min(t + u, depth - 1) * SLICE)[lane];
+#pragma unroll
+            for (int u = 0; u < US; ++u)
+                if (t + u < count) surface += m[u];
+        }
+        tiny = 1e-6 * surface;
+    }
+    {
+        // The list walk: while entry t is summed, the rows of entry t + 1 are on their way to LDS and those of entry t + 2
+        // asked for. Every lane takes part in every fetch; the list's padding names cell 0, and past the end the last
+        // entry is fetched again, so that two fetches are always in flight.
+        Stage<D> stage;
+        stage.init(lane, lds);
+        const int last = depth - 1;
+        if (depth > 0) {
+            int next = (other + min(2, last) * SLICE)[lane];
+            stage.address(other[lane]);
+            stage.fetch(g.cell, 0);
+            stage.address((other + min(1, last) * SLICE)[lane]);
+            stage.fetch(g.cell, 1);
+            double mag = geometry[lane];
+            stage.address(next);
+            next = (other + min(3, last) * SLICE)[lane];
+            for (int t = 0; t < depth; ++t) {
+                Near<D> n;
+                stage.read(t & 1, n);
+                n.mag = mag;
+                mag = (geometry + min(t + 1, last) * SLICE)[lane];
+                const int after = (other + min(t + 4, last) * SLICE)[lane];
+                stage.fetch(g.cell, t & 1);  // the last loads of the iteration: read() counts on it
+                stage.address(next);
+                next = after;
+                if (t < count) s.add(g, n, xi, centroid, Wi, ci, ri, courant, tiny);
+            }
+            stage.drain();
+        }
+    }
+    smallest = s.smallest;
+    bool ok = s.ok;
+    G grad[V][D], intercept[V];
+    if constexpr (Grad) {  // Sweep::solve (:590-615): Cholesky of M, then M x = b per variable
+        G L[U][U];
+        Divisor by[U];
+#pragma unroll
+        for (int p = 0; p < U; ++p)
+#pragma unroll
+            for (int q = 0; q <= p; ++q) {
+                G sum = s.M[q][p];
+#pragma unroll
+                for (int m = 0; m < q; ++m) sum -= L[p][m] * L[q][m];
+                if constexpr (exact) {
+                    L[p][q] = p == q ? Op::square_root(sum) : Op::quotient(sum, by[q]);
+                    if (p == q) {
+                        by[p] = Op::by(L[p][p]);
+                        if constexpr (Fast) ok = ok && plain(L[p][p]);
+                    }
+                } else {
+                    L[p][q] = p == q ? sqrt(sum) : sum / L[q][q];
+                }
+            }
+        auto divide = [&](G a, int p) -> G {
+            if constexpr (exact)
+                return Op::quotient(a, by[p]);
+            else
+                return a / L[p][p];
+        };
+        G size = 0;
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            G z[U], x[U];
+#pragma unroll
+            for (int p = 0; p < U; ++p) {
+                G sum = s.b[v][p];
+#pragma unroll
+                for (int m = 0; m < p; ++m) sum -= L[p][m] * z[m];
+                z[p] = divide(sum, p);
+            }
+#pragma unroll
+            for (int p = U - 1; p >= 0; --p) {
+                G sum = z[p];
+#pragma unroll
+                for (int m = p + 1; m < U; ++m) sum -= L[m][p] * x[m];
+                x[p] = divide(sum, p);
+                if constexpr (Fast && exact) size += fabs(x[p]);
+            }
+#pragma unroll
+            for (int a = 0; a < D; ++a) grad[v][a] = x[1 + a];
+            intercept[v] = x[0];
+        }
+        if constexpr (Fast && exact) ok = ok && size < 0x1p900;  // an overflow on the way leaves a NaN in some x
+    }
+    double wi[D];
+#pragma unroll
+    for (int a = 0; a < D; ++a) wi[a] = Wi[1 + a];
+    if constexpr (Moving) {  // the regularised point velocity (:526-537; constants :74)
+        const double shaping = 0.5, factor = 2.25;
+        double fraction = 0;
+        if (s.max_angle > 0.75 * factor)
+            fraction = s.max_angle > factor ? shaping : shaping * (s.max_angle - 0.75 * factor) / (0.25 * factor);
+        const double cd = sqrt(dot<D>(centroid, centroid));
+        if (cd > 0 && fraction > 0) {
+            const double sc = fraction * ci / cd;
+#pragma unroll
+            for (int a = 0; a < D; ++a) wi[a] = wi[a] + centroid[a] * sc;
+        }
+    }
+    if constexpr (Rule == 0) {  // CellStep (:1046-1051)
+        double rel[D];
+#pragma unroll
+        for (int a = 0; a < D; ++a) rel[a] = Moving ? Wi[1 + a] - wi[a] : Wi[1 + a];
+        const double step = ri / (ci + sqrt(dot<D>(rel, rel)));
+        smallest = fmin(smallest, courant * step);
+    } else {  // LunaStep (:1061-1070), 2D
+        const double dx = ri * sqrt(M_PI);
+        double rate = 0;
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            double relative = Wi[1 + a];
+            if constexpr (Moving) relative -= wi[a];
+            rate += (fabs(relative) + ci) / dx;
+        }
+        smallest = fmin(smallest, courant / rate);
+    }
+    [[maybe_unused]] Record<D, Limit == 2> rec;
+    if constexpr (Grad && Limit > 0) {  // the face-centroid limiter, face by face in list order (:538-565)
+        if constexpr (Fast && exact) {  // the rooms the clips divide by the change: none too small for over()
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                const double up = s.hi[v] - Wi[v], down = Wi[v] - s.lo[v];
+                ok = ok && (!(up > 0) || up > 0x1p-900) && (!(down > 0) || down > 0x1p-900);
+            }
+        }
+        // Geometry::face_offset (:322-326), kept per slot, of UL entries loaded together, then applied in order. A face
+        // clips the variables it must in one pass over all of them without branches (a factor of 1 leaves a gradient as it
+        // is), so their divisions run side by side.
+        constexpr int UL = LUNA_LIMIT_UNROLL;
+        if constexpr (exact) rec.init(grad);
+        for (int t0 = 0; t0 < depth; t0 += UL) {
+            double offset[UL][D], mag[UL];
+#pragma unroll
+            for (int u = 0; u < UL; ++u) {
+                const double* entry = geometry + min(t0 + u, depth - 1) * SLICE;
+                mag[u] = entry[lane];
+#pragma unroll
+                for (int a = 0; a < D; ++a) offset[u][a] = (entry + (a + 1) * g.slots)[lane];
+            }
+#pragma unroll
+            for (int u = 0; u < UL; ++u) {
+                const bool use = t0 + u < count && !(mag[u] < tiny);
+                if constexpr (exact) {
+                    double dp[V], bound[V];
+                    bool clip[V], any = false;
+#pragma unroll
+                    for (int v = 0; v < V; ++v) {
+                        dp[v] = dot<D>(grad[v], offset[u]);
+                        const double at = Wi[v] + dp[v];
+                        const bool up = dp[v] > 0 && at > s.hi[v], down = dp[v] < 0 && at < s.lo[v];
+                        clip[v] = use && (up || down);
+                        bound[v] = dp[v] > 0 ? s.hi[v] : s.lo[v];
+                        any = any || clip[v];
+                    }
+                    if (use) rec.face(offset[u]);
+                    if (__any(any)) {
+#pragma unroll
+                        for (int v = 0; v < V; ++v) {
+                            // (bound - W) / dp where the bound is on the change's side of W, else 0
+                            const double q = Op::quotient(bound[v] - Wi[v], Op::by(dp[v]));
+                            const double sc = clip[v] ? (q > 0 ? q : 0.0) : 1.0;
+#pragma unroll
+                            for (int a = 0; a < D; ++a) grad[v][a] = grad[v][a] * sc;
+                            if (clip[v]) rec.clip(v, sc);
+                        }
+                    }
+                } else {  // reduced precision (:558-562): the offset, the face's change and the range relative to W_i in G
+                    if (!use) continue;
+                    G rg[D];
+#pragma unroll
+                    for (int a = 0; a < D; ++a) rg[a] = (G)offset[u][a];
+#pragma unroll
+                    for (int v = 0; v < V; ++v) {
+                        const G dp = dot<D>(grad[v], rg);
+                        if (dp > 0 && dp > s.hi[v]) {
+                            const G sc = s.hi[v] > 0 ? s.hi[v] / dp : G(0);
+#pragma unroll
+                            for (int a = 0; a < D; ++a) grad[v][a] = grad[v][a] * sc;
+                        } else if (dp < 0 && dp < s.lo[v]) {
+                            const G sc = s.lo[v] < 0 ? s.lo[v] / dp : G(0);
+#pragma unroll
+                            for (int a = 0; a < D; ++a) grad[v][a] = grad[v][a] * sc;
+                        }
+                    }
+                }
+            }
+        }
+    }
+    if constexpr (Fast) {
+        if (!__all(ok || !here)) return false;
+    }
+    if (!here) {
+        smallest = INFINITY;
+        return true;
+    }
+    if constexpr (Moving) {
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            r.w[(size_t)i * D + a] = wi[a];
+            r.old_centroid[(size_t)i * D + a] = centroid[a];  // keep_centroids (:1506-1514): c^n for the second pass
+        }
+    }
+    if constexpr (Limit == 2 && exact) {
+        Cell<D> cell;
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            cell.W[v] = Wi[v];
+            cell.lo[v] = s.lo[v];
+            cell.hi[v] = s.hi[v];
+            cell.intercept[v] = intercept[v];
+        }
+        cell.cs = ci;
+        cell.r = ri;
+        cell.count = count;
+        r.troubled[i] = limiter_features<D>(cell, rec, r.features + (size_t)i * V * FEATURES);
+    }
+    if constexpr (Grad) {
+        store_gradient<D, Prec>(r, i, grad);
+        if constexpr (exact && Limit < 2) {
+            if (r.hll) {  // the compression indicator of the HLL fallback
+                double div = 0;
+#pragma unroll
+                for (int a = 0; a < D; ++a) div += grad[1 + a][a];
+                r.hll[i] = div * ri / ci < -r.hll_threshold ? 1 : 0;
+            }
+        }
+    }
+    return true;
+}
+
+// The first block also resets the other dt slot and the step's fallback counters.
+template <int D, bool Moving, bool Grad, int Limit, int Rule, int Prec = 0>
+__global__ __launch_bounds__(CELL_BLOCK, Limit == 2 ? 1 : LUNA_SWEEP_WAVES) void k_sweep(Geo g, Rows r, Gas gas, double courant, Counters c) {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         *c.dt_next = INF_BITS;
         c.fallbacks[0] = 0;
         c.fallbacks[1] = 0;
     }
+    __shared__ double rows[Stage<D>::DOUBLES];
+    lds_double* lds = (lds_double*)rows;
+    const int block = xcd_block();
     double smallest = INFINITY;
-    if (i < g.N) {
-        const double* mine = g.cell + (size_t)i * CELL_ROW;
-        double Wi[V], xi[D], centroid[D];
-#pragma unroll
-        for (int v = 0; v < V; ++v) Wi[v] = mine[C::W + v];
-        const double ci = mine[C::CS], ri = mine[C::RAD];
-        load_vec<D>(mine + C::X, xi);
-        load_vec<D>(mine + C::C, centroid);
-        constexpr bool range_pass = LUNA_RANGE_PASS || (Moving && exact);  // the float sums fit 3 waves without it
-        Sums<D, Moving, Grad, Rule, G, range_pass> s;
-        s.init();
-        const int count = g.count[i], base = first_slot(g, i);
-        // Groups of UN entries: their face magnitudes and rows in flight together, summed in list order; the next group's
-        // other-cell indices are read one group ahead, so each group waits for one level of loads.
-        constexpr int UN = exact ? LUNA_SWEEP_UNROLL : 2;
-        int nj[UN];
-#pragma unroll
-        for (int u = 0; u < UN; ++u)
-            if (u < count) nj[u] = g.other[base + u * SLICE];
-        int t = 0;
-        for (; t + UN - 1 < count; t += UN) {
-            int cj[UN];
-#pragma unroll
-            for (int u = 0; u < UN; ++u) {
-                cj[u] = nj[u];
-                if (t + UN + u < count) nj[u] = g.other[base + (t + UN + u) * SLICE];
-            }
-            Near<D> n[UN];
-#pragma unroll
-            for (int u = 0; u < UN; ++u) load_near<D>(g, base + (t + u) * SLICE, cj[u], n[u]);
-#pragma unroll
-            for (int u = 0; u < UN; ++u) s.add(g, n[u], xi, centroid, Wi, ci, ri, courant);
-        }
-#pragma unroll
-        for (int u = 0; u < UN - 1; ++u)
-            if (t + u < count) {
-                Near<D> a;
-                load_near<D>(g, base + (t + u) * SLICE, nj[u], a);
-                s.add(g, a, xi, centroid, Wi, ci, ri, courant);
-            }
-        smallest = s.smallest;
-        const double tiny = 1e-6 * s.surface;
-        const bool any_tiny = s.smallest_face < tiny;
-        // neighbour_range (:572-588): the range of the neighbours' W, faces under 1e-6 of the surface left out if any
-        auto neighbour_range = [&]() {
-#pragma unroll
-            for (int v = 0; v < V; ++v) {
-                s.lo[v] = finite_max<G>();
-                s.hi[v] = -finite_max<G>();
-            }
-            for (int k = 0; k < count; ++k) {
-                if (any_tiny && g.slot[base + k * SLICE] < tiny) continue;
-                const double* row = g.cell + (size_t)g.other[base + k * SLICE] * CELL_ROW + C::W;
-#pragma unroll
-                for (int v = 0; v < V; ++v) {
-                    const G value = exact ? (G)row[v] : (G)(row[v] - Wi[v]);
-                    s.lo[v] = fmin(s.lo[v], value);
-                    s.hi[v] = fmax(s.hi[v], value);
-                }
-            }
-        };
-        if constexpr (Grad && !range_pass) {
-            if (any_tiny) neighbour_range();
-        }
-        G grad[V][D], intercept[V];
-        if constexpr (Grad) {  // Sweep::solve (:590-615): Cholesky of M, then M x = b per variable
-            G L[U][U];
-#pragma unroll
-            for (int p = 0; p < U; ++p)
-#pragma unroll
-                for (int q = 0; q < U; ++q) L[p][q] = 0;
-#pragma unroll
-            for (int p = 0; p < U; ++p)
-#pragma unroll
-                for (int q = 0; q <= p; ++q) {
-                    G sum = s.M[q][p];
-#pragma unroll
-                    for (int m = 0; m < q; ++m) sum -= L[p][m] * L[q][m];
-                    L[p][q] = p == q ? sqrt(sum) : sum / L[q][q];
-                }
-#pragma unroll
-            for (int v = 0; v < V; ++v) {
-                G z[U], x[U];
-#pragma unroll
-                for (int p = 0; p < U; ++p) {
-                    G sum = s.b[v][p];
-#pragma unroll
-                    for (int m = 0; m < p; ++m) sum -= L[p][m] * z[m];
-                    z[p] = sum / L[p][p];
-                }
-#pragma unroll
-                for (int p = U - 1; p >= 0; --p) {
-                    G sum = z[p];
-#pragma unroll
-                    for (int m = p + 1; m < U; ++m) sum -= L[m][p] * x[m];
-                    x[p] = sum / L[p][p];
-                }
-#pragma unroll
-                for (int a = 0; a < D; ++a) grad[v][a] = x[1 + a];
-                intercept[v] = x[0];
-            }
-        }
-        double wi[D];
-#pragma unroll
-        for (int a = 0; a < D; ++a) wi[a] = Wi[1 + a];
-        if constexpr (Moving) {  // the regularised point velocity (:526-537; constants :74)
-            const double shaping = 0.5, factor = 2.25;
-            double fraction = 0;
-            if (s.max_angle > 0.75 * factor)
-                fraction = s.max_angle > factor ? shaping : shaping * (s.max_angle - 0.75 * factor) / (0.25 * factor);
-            const double cd = sqrt(dot<D>(centroid, centroid));
-            if (cd > 0 && fraction > 0) {
-                const double sc = fraction * ci / cd;
-#pragma unroll
-                for (int a = 0; a < D; ++a) wi[a] = wi[a] + centroid[a] * sc;
-            }
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-                r.w[(size_t)i * D + a] = wi[a];
-                r.old_centroid[(size_t)i * D + a] = centroid[a];  // keep_centroids (:1506-1514): c^n for the second pass
-            }
-        }
-        if constexpr (Rule == 0) {  // CellStep (:1046-1051)
-            double rel[D];
-#pragma unroll
-            for (int a = 0; a < D; ++a) rel[a] = Moving ? Wi[1 + a] - wi[a] : Wi[1 + a];
-            const double step = ri / (ci + sqrt(dot<D>(rel, rel)));
-            smallest = fmin(smallest, courant * step);
-        } else {  // LunaStep (:1061-1070), 2D
-            const double dx = ri * sqrt(M_PI);
-            double rate = 0;
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-                double relative = Wi[1 + a];
-                if constexpr (Moving) relative -= wi[a];
-                rate += (fabs(relative) + ci) / dx;
-            }
-            smallest = fmin(smallest, courant / rate);
-        }
-        if constexpr (Grad) {
-            if constexpr (Limit > 0 && range_pass) neighbour_range();
-            if constexpr (Limit > 0) {  // the face-centroid limiter, face by face in list order (:538-565)
-                // Geometry::face_offset (:322-326), kept per slot, of UL entries loaded together, then applied in order.
-                constexpr int UL = LUNA_LIMIT_UNROLL;
-                Record<D, Limit == 2> rec;
-                if constexpr (exact) rec.init(grad);
-                for (int t2 = 0; t2 < count; t2 += UL) {
-                    double offset[UL][D];
-                    bool use[UL];
-#pragma unroll
-                    for (int u = 0; u < UL; ++u) {
-                        use[u] = false;
-                        if (t2 + u < count) {
-                            const long long slot = base + (t2 + u) * SLICE;
-                            use[u] = !(any_tiny && g.slot[slot] < tiny);
-#pragma unroll
-                            for (int a = 0; a < D; ++a) offset[u][a] = g.slot[(a + 1) * g.slots + slot];
-                        }
-                    }
-#pragma unroll
-                    for (int u = 0; u < UL; ++u) {
-                        if (!use[u]) continue;
-                        if constexpr (exact) {
-                            rec.face(offset[u]);
-#pragma unroll
-                            for (int v = 0; v < V; ++v) {
-                                const double dp = dot<D>(grad[v], offset[u]);
-                                if (dp > 0 && Wi[v] + dp > s.hi[v]) {
-                                    const double sc = s.hi[v] > Wi[v] ? (s.hi[v] - Wi[v]) / dp : 0.0;
-#pragma unroll
-                                    for (int a = 0; a < D; ++a) grad[v][a] = grad[v][a] * sc;
-                                    rec.clip(v, sc);
-                                } else if (dp < 0 && Wi[v] + dp < s.lo[v]) {
-                                    const double sc = s.lo[v] < Wi[v] ? (s.lo[v] - Wi[v]) / dp : 0.0;
-#pragma unroll
-                                    for (int a = 0; a < D; ++a) grad[v][a] = grad[v][a] * sc;
-                                    rec.clip(v, sc);
-                                }
-                            }
-                        } else {  // reduced precision (:558-562): the offset, the face's change and the range relative to W_i in G
-                            G rg[D];
-#pragma unroll
-                            for (int a = 0; a < D; ++a) rg[a] = (G)offset[u][a];
-#pragma unroll
-                            for (int v = 0; v < V; ++v) {
-                                const G dp = dot<D>(grad[v], rg);
-                                if (dp > 0 && dp > s.hi[v]) {
-                                    const G sc = s.hi[v] > 0 ? s.hi[v] / dp : G(0);
-#pragma unroll
-                                    for (int a = 0; a < D; ++a) grad[v][a] = grad[v][a] * sc;
-                                } else if (dp < 0 && dp < s.lo[v]) {
-                                    const G sc = s.lo[v] < 0 ? s.lo[v] / dp : G(0);
-#pragma unroll
-                                    for (int a = 0; a < D; ++a) grad[v][a] = grad[v][a] * sc;
-                                }
-                            }
-                        }
-                    }
-                }
-                if constexpr (Limit == 2 && exact) {
-                    Cell<D> cell;
-#pragma unroll
-                    for (int v = 0; v < V; ++v) {
-                        cell.W[v] = Wi[v];
-                        cell.lo[v] = s.lo[v];
-                        cell.hi[v] = s.hi[v];
-                        cell.intercept[v] = intercept[v];
-                    }
-                    cell.cs = ci;
-                    cell.r = ri;
-                    cell.count = count;
-                    r.troubled[i] = limiter_features<D>(cell, rec, r.features + (size_t)i * V * FEATURES);
-                }
-            }
-            store_gradient<D, Prec>(r, i, grad);
-            if constexpr (exact && Limit < 2) {
-                if (r.hll) {  // the compression indicator of the HLL fallback
-                    double div = 0;
-#pragma unroll
-                    for (int a = 0; a < D; ++a) div += grad[1 + a][a];
-                    r.hll[i] = div * ri / ci < -r.hll_threshold ? 1 : 0;
-                }
-            }
-        }
-    }
+    if (!sweep_slice<D, Moving, Grad, Limit, Rule, Prec, true>(g, r, courant, block, lds, smallest))
+        sweep_slice<D, Moving, Grad, Limit, Rule, Prec, false>(g, r, courant, block, lds, smallest);
     block_min<CELL_BLOCK>(smallest, c.dt);
 }
 
@@ -583,16 +756,19 @@ __global__ __launch_bounds__(CELL_BLOCK, LUNA_LANE_WAVES(L)) void k_sweep_lanes(
         const double ci = mine[C::CS], ri = mine[C::RAD];
         load_vec<D>(mine + C::X, xi);
         load_vec<D>(mine + C::C, centroid);
-        Sums<D, Moving, true, Rule, double, false> s;
+        Sums<D, Moving, true, Rule, double> s;
         s.init();
+        double surface = 0, smallest_face = INFINITY;
         const int count = g.count[i], base = first_slot(g, i);
         for (int t = lane; t < count; t += L) {
             Near<D> n;
             load_near<D>(g, base + t * SLICE, g.other[base + t * SLICE], n);
-            s.add(g, n, xi, centroid, Wi, ci, ri, courant);
+            surface += n.mag;
+            smallest_face = fmin(smallest_face, n.mag);
+            s.add(g, n, xi, centroid, Wi, ci, ri, courant, 0.0);
         }
-        s.surface = lanes_sum<L>(s.surface);
-        s.smallest_face = lanes_min<L>(s.smallest_face);
+        surface = lanes_sum<L>(surface);
+        smallest_face = lanes_min<L>(smallest_face);
         if constexpr (Moving) s.max_angle = lanes_max<L>(s.max_angle);
         smallest = lanes_min<L>(s.smallest);
 #pragma unroll
@@ -606,8 +782,8 @@ __global__ __launch_bounds__(CELL_BLOCK, LUNA_LANE_WAVES(L)) void k_sweep_lanes(
             s.lo[v] = lanes_min<L>(s.lo[v]);
             s.hi[v] = lanes_max<L>(s.hi[v]);
         }
-        const double tiny = 1e-6 * s.surface;
-        const bool any_tiny = s.smallest_face < tiny;
+        const double tiny = 1e-6 * surface;
+        const bool any_tiny = smallest_face < tiny;
         if (any_tiny) {  // rare: the range again without the tiny faces, each lane walking the whole list
 #pragma unroll
             for (int v = 0; v < V; ++v) {

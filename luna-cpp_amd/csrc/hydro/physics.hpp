@@ -6,6 +6,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "exact_math.hpp"
+
 namespace luna {
 
 struct Gas {
@@ -274,6 +276,6 @@ __device__ __forceinline__ void riemann(int kind, const Gas& gas, const double* 
 
 // The nearest periodic image of a separation, given the box side and its inverse (the role of tet_mesh::wrap(d, side,
 // inverse) in Geometry::separation, finite_volume.hpp:279-282).
-__device__ __forceinline__ double wrap(double d, double side, double inverse) { return d - side * round(d * inverse); }
+__device__ __forceinline__ double wrap(double d, double side, double inverse) { return d - side * round_half_away(d * inverse); }
 
 }  // namespace luna
