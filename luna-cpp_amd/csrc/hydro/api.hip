@@ -153,7 +153,7 @@ struct luna_fv {
     Buf<double> q, grad, w, x, old_centroid, flux;
     Buf<unsigned int> exponents;  // grad16: the per-cell group exponents (int8 x 3)
     Buf<unsigned char> hll;       // the HLL fallback's per-cell compression flags
-    Buf<unsigned long long> counters;  // [0, 1] dt slots, [2, 3] fallbacks of the step's two flux passes
+    Buf<unsigned long long> counters;  // two sets of dt slots, then the fallbacks of the step's two flux passes
     // the derivatives' rows (first use): luna::Derivs
     Buf<double> d_dq, d_dW, d_dgrad, d_dflux, d_sidebar, d_bbar, d_boundbar, d_out;
     Buf<int> d_extreme;
@@ -222,7 +222,9 @@ struct luna_fv {
     }
     luna::Gas gas() const { return luna::Gas{opt.gamma, opt.smallr, opt.smallc, 1.0 / (opt.gamma - 1.0)}; }
     luna::Counters counters_now() const {
-        return luna::Counters{counters.p + parity, counters.p + (parity ^ 1), counters.p + 2};
+        return luna::Counters{counters.p + parity * luna::DT_WORDS, counters.p + (parity ^ 1) * luna::DT_WORDS, fallback_counters()};
+    }
+    unsigned long long* fallback_counters() const { return counters.p + 2 * luna::DT_WORDS;
     }
 };
 
@@ -455,6 +457,19 @@ int sweep(luna_fv* fv, double courant, bool dt_only = false) {
     return LUNA_OK;
 }
 
+// The time step of the sweep that wrote the dt slots of `parity`: their smallest, read back (blocks).
+int read_time_step(luna_fv* fv, int parity, double* dt) {
+    unsigned long long* slots = fv->host + 8;
+    LUNA_HIP(hipMemcpyAsync(slots, fv->counters.p + parity * luna::DT_WORDS, sizeof(unsigned long long) * luna::DT_WORDS, hipMemcpyDeviceToHost,
+                            fv->stream));
+    LUNA_HIP(hipStreamSynchronize(fv->stream));
+    LUNA_HIP(fv->prof.collect());
+    unsigned long long least = luna::INF_BITS;
+    for (int k = 0; k < luna::DT_SLOTS; ++k) least = std::min(least, slots[k * luna::DT_STRIDE]);
+    *dt = bits_to_double(least);
+    return LUNA_OK;
+}
+
 int ensure_swept(luna_fv* fv) {
     if (!fv->mesh_ok) return fail(LUNA_ERR_LOGIC, "luna: the last mesh given was refused; set a valid mesh first");
     if (fv->swept) return LUNA_OK;
@@ -472,7 +487,7 @@ int flux_and_update(luna_fv* fv, int pass, double flux_dt, double apply_dt, doub
     const luna::Rows r = fv->rows();
     const luna::Gas gas = fv->gas();
     hipStream_t s = fv->stream;
-    unsigned long long* count = fv->counters.p + (pass == 1 ? 3 : 2);
+    unsigned long long* count = fv->fallback_counters() + (pass == 1 ? 1 : 0);
     const int riemann = fv->riemann(), order = fv->opt.order;
     if (prims) *prims = next_prims && fv->opt.update != LUNA_UPDATE_PER_CELL;
     if (fv->opt.update == LUNA_UPDATE_PER_CELL) {
@@ -552,7 +567,7 @@ int create(const luna_fv_options* opt, const luna_geometry* mesh, luna_fv** out,
     if ((e = fv->q.reserve(N * V)) != hipSuccess || (e = fv->count.reserve(N)) != hipSuccess ||
         (e = fv->grad.reserve(N * fv->grad_row())) != hipSuccess || (e = fv->w.reserve(N * D)) != hipSuccess ||
         (e = fv->cell.reserve(N * luna::CELL_ROW)) != hipSuccess || (e = fv->volume.reserve(N)) != hipSuccess ||
-        (e = fv->counters.reserve(4)) != hipSuccess || (e = fv->geo_info.reserve(1)) != hipSuccess ||
+        (e = fv->counters.reserve(2 * luna::DT_WORDS + 2)) != hipSuccess || (e = fv->geo_info.reserve(1)) != hipSuccess ||
         (e = fv->geo_flags.reserve(1)) != hipSuccess)
         return cleanup(fail(LUNA_ERR_MEMORY, std::string("luna: device allocation: ") + hipGetErrorString(e)));
     if (opt->limiter == LUNA_LIMITER_LEARNED) {
@@ -569,10 +584,11 @@ int create(const luna_fv_options* opt, const luna_geometry* mesh, luna_fv** out,
             (e = fv->steps.reserve(N * D)) != hipSuccess)
             return cleanup(fail(LUNA_ERR_MEMORY, std::string("luna: device allocation: ") + hipGetErrorString(e)));
     }
-    if (hipHostMalloc(reinterpret_cast<void**>(&fv->host), 8 * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess)
+    if (hipHostMalloc(reinterpret_cast<void**>(&fv->host), (8 + luna::DT_WORDS) * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess)
         return cleanup(fail(LUNA_ERR_MEMORY, "luna: pinned host allocation failed"));
-    const unsigned long long init[4] = {luna::INF_BITS, luna::INF_BITS, 0, 0};
-    if (hipMemcpy(fv->counters.p, init, sizeof init, hipMemcpyHostToDevice) != hipSuccess)
+    std::vector<unsigned long long> init(2 * luna::DT_WORDS + 2, luna::INF_BITS);
+    init[2 * luna::DT_WORDS] = init[2 * luna::DT_WORDS + 1] = 0;
+    if (hipMemcpy(fv->counters.p, init.data(), sizeof(unsigned long long) * init.size(), hipMemcpyHostToDevice) != hipSuccess)
         return cleanup(fail(LUNA_ERR_DEVICE, "luna: counter initialisation failed"));
     std::vector<double> zero(N * V, 0.0);
     if (hipMemcpy(fv->q.p, zero.data(), sizeof(double) * N * V, hipMemcpyHostToDevice) != hipSuccess)
@@ -662,10 +678,7 @@ int luna_fv_time_step(luna_fv* fv, double courant, double* dt) {
     fv->prims_ready = false;
     const int slot = fv->parity;
     if (int rc = sweep(fv, courant)) return rc;
-    LUNA_HIP(hipMemcpyAsync(fv->host, fv->counters.p + slot, sizeof(unsigned long long), hipMemcpyDeviceToHost, fv->stream));
-    LUNA_HIP(hipStreamSynchronize(fv->stream));
-    LUNA_HIP(fv->prof.collect());
-    *dt = bits_to_double(fv->host[0]);
+    if (int rc = read_time_step(fv, slot, dt)) return rc;
     fv->swept = true;
     fv->tangent_swept = false;
     return LUNA_OK;
@@ -762,10 +775,7 @@ int luna_fv_time_step_tangent(luna_fv* fv, double courant, const double* dq, int
     LUNA_HIP(timed(fv->prof, s, "sweep_tangent", [&] {
         return fv->D == 3 ? luna::launch_sweep_tangent<3>(s, g, r, gas, limit, w) : luna::launch_sweep_tangent<2>(s, g, r, gas, limit, w);
     }));
-    LUNA_HIP(hipMemcpyAsync(fv->host, fv->counters.p + slot, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-    LUNA_HIP(hipStreamSynchronize(s));
-    LUNA_HIP(fv->prof.collect());
-    *dt = bits_to_double(fv->host[0]);
+    if (int rc = read_time_step(fv, slot, dt)) return rc;
     fv->swept = true;
     fv->tangent_swept = true;
     return LUNA_OK;
@@ -1227,7 +1237,7 @@ int luna_synchronize(void) {
 
 int luna_fv_fallbacks(luna_fv* fv, long long* count) {
     if (!fv || !count) return fail(LUNA_ERR_ARGUMENT, "luna_fv_fallbacks: null argument");
-    LUNA_HIP(hipMemcpyAsync(fv->host + 2, fv->counters.p + 2, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, fv->stream));
+    LUNA_HIP(hipMemcpyAsync(fv->host + 2, fv->fallback_counters(), 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, fv->stream));
     LUNA_HIP(hipStreamSynchronize(fv->stream));
     LUNA_HIP(fv->prof.collect());
     *count = static_cast<long long>(fv->host[2] + fv->host[3]);

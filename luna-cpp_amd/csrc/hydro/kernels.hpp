@@ -113,9 +113,13 @@ struct Grid {
     long long period[3];
 };
 
+// The mesh sweeps' min-reduction goes to DT_SLOTS addresses a cache line apart (work-group b to slot b mod DT_SLOTS), whose
+// smallest the host takes: atomics to one address are served one after the other, about 11 ns each on MI355X, so that the
+// 4096 wavefronts of a 511^2 sweep took 76 us with one address and take 38 with 32. (A line's kernels use the first alone.)
+constexpr int DT_SLOTS = 32, DT_STRIDE = 16, DT_WORDS = DT_SLOTS * DT_STRIDE;
 struct Counters {
     unsigned long long* dt;         // the min-reduction this sweep writes
-    unsigned long long* dt_next;    // the other slot, reset for the next sweep
+    unsigned long long* dt_next;    // the other one, reset for the next sweep
     unsigned long long* fallbacks;  // [2]: face sides that took the cell's state, per flux pass of the step
 };
 

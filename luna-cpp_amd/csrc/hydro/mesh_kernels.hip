@@ -72,6 +72,12 @@ __device__ __forceinline__ void block_min(double v, unsigned long long* out) {
         if (m < INFINITY) atomicMin(out, (unsigned long long)__double_as_longlong(m));
     }
 }
+// The first block resets the other dt slots and the step's fallback counters.
+__device__ __forceinline__ void reset_counters(const Counters& c) {
+    if (blockIdx.x != 0) return;
+    if (threadIdx.x < DT_SLOTS) c.dt_next[threadIdx.x * DT_STRIDE] = INF_BITS;
+    if (threadIdx.x < 2) c.fallbacks[threadIdx.x] = 0;
+}
 template <int B>
 __device__ __forceinline__ void block_count(int v, unsigned long long* out) {
     __shared__ int part[B / 64];
@@ -693,21 +699,16 @@ __device__ __forceinline__ bool sweep_slice(const Geo& g, const Rows& r, double 
     return true;
 }
 
-// The first block also resets the other dt slot and the step's fallback counters.
 template <int D, bool Moving, bool Grad, int Limit, int Rule, int Prec = 0>
 __global__ __launch_bounds__(CELL_BLOCK, Limit == 2 ? 1 : LUNA_SWEEP_WAVES) void k_sweep(Geo g, Rows r, Gas gas, double courant, Counters c) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        *c.dt_next = INF_BITS;
-        c.fallbacks[0] = 0;
-        c.fallbacks[1] = 0;
-    }
+    reset_counters(c);
     __shared__ double rows[Stage<D>::DOUBLES];
     lds_double* lds = (lds_double*)rows;
     const int block = xcd_block();
     double smallest = INFINITY;
     if (!sweep_slice<D, Moving, Grad, Limit, Rule, Prec, true>(g, r, courant, block, lds, smallest))
         sweep_slice<D, Moving, Grad, Limit, Rule, Prec, false>(g, r, courant, block, lds, smallest);
-    block_min<CELL_BLOCK>(smallest, c.dt);
+    block_min<CELL_BLOCK>(smallest, c.dt + (blockIdx.x % DT_SLOTS) * DT_STRIDE);
 }
 
 // finite_volume.hpp:880-1037 LaneSweep: L lanes per cell (L = 2, 4 or 8; 64 / L cells per wavefront). Lane l takes the
@@ -742,11 +743,7 @@ __global__ __launch_bounds__(CELL_BLOCK, LUNA_LANE_WAVES(L)) void k_sweep_lanes(
     using C = CellAt<D>;
     const int lane = threadIdx.x & (L - 1);
     const int i = xcd_block() * CELLS + threadIdx.x / L;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        *c.dt_next = INF_BITS;
-        c.fallbacks[0] = 0;
-        c.fallbacks[1] = 0;
-    }
+    reset_counters(c);
     double smallest = INFINITY;
     if (i < g.N) {  // the same for the L lanes of a cell, so their shuffles stay among active lanes
         const double* mine = g.cell + (size_t)i * CELL_ROW;
@@ -915,7 +912,7 @@ __global__ __launch_bounds__(CELL_BLOCK, LUNA_LANE_WAVES(L)) void k_sweep_lanes(
             }
         }
     }
-    block_min<CELL_BLOCK>(smallest, c.dt);
+    block_min<CELL_BLOCK>(smallest, c.dt + (blockIdx.x % DT_SLOTS) * DT_STRIDE);
 }
 
 // finite_volume.hpp:1306-1329 FaceFlux::side() at order 1: half step (over step_dt) + g.r, positivity fallback. prow,
