@@ -143,14 +143,15 @@ __device__ __forceinline__ void load_near(const Geo& g, int slot, int j, Near<D>
     n.cs = row[C::CS];
 }
 
+typedef __attribute__((address_space(3))) double lds_double;
+typedef double double2v __attribute__((ext_vector_type(2)));
+
 // A wavefront's neighbour rows through LDS. A lane that loads its own neighbour's row itself touches a 128 B line per 16 B
 // load, and a CU's L1 looks up one line a cycle: the rows of 64 neighbours cost 7 x 64 lookups, which bound the list walk
 // (5.6 thousand cycles an entry at 12 wavefronts a CU). Here the 16 B chunks of all 64 rows are dealt to the lanes in order
 // (chunk q to lane q mod 64 of load q / 64, of row q / CHUNKS), so that a load covers whole rows, and go to LDS without
 // passing through registers, back to back (a row at 16 CHUNKS bytes times its lane). Chunks with neither x, c, W nor c_s
 // (V and r) are skipped. Two buffers: one is read while the other is in flight.
-typedef __attribute__((address_space(3))) double lds_double;
-typedef double double2v __attribute__((ext_vector_type(2)));
 template <int D>
 struct Stage {
     static constexpr int CHUNKS = D == 3 ? 6 : 5, ROW = 2 * CHUNKS;  // a staged row: [x, c, W, c_s]
@@ -275,23 +276,34 @@ __device__ __forceinline__ void store_gradient(const Rows& r, int i, const G (&g
                          (unsigned)(unsigned char)(signed char)k[2] << 16;
     }
 }
-// The gradient row of cell i in float (reduced-precision policies), decoded from FP16 if need be (FaceFlux::gradient,
-// :1288-1300).
-template <int D, int Prec>
-__device__ __forceinline__ void load_gradient_lp(const Rows& r, int i, float* gr) {
+// A gradient row in float (reduced-precision policies), decoded from FP16 with the cell's exponents k if need be
+// (FaceFlux::gradient, :1288-1300). Row: the row's 16 B chunks by number.
+template <int D, int Prec, class Row>
+__device__ __forceinline__ void decode_gradient(const Row& chunk, unsigned k, float* gr) {
     constexpr int VD = (D + 2) * D;
     if constexpr (Prec == 1) {
-        const float* p = reinterpret_cast<const float*>(r.grad) + (size_t)i * lp_row<D>();
 #pragma unroll
-        for (int c = 0; c < VD; ++c) gr[c] = p[c];
+        for (int c = 0; c < VD; c += 4) {
+            const double2v d = chunk(c / 4);
+            float v[4];
+            __builtin_memcpy(v, &d, 16);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (c + e < VD) gr[c + e] = v[e];
+        }
     } else {
-        const unsigned short* p = reinterpret_cast<const unsigned short*>(r.grad) + (size_t)i * HALF_ROW;
-        const unsigned k = r.exponents[i];
         float scale[3];
 #pragma unroll
         for (int q = 0; q < 3; ++q) scale[q] = power_of_two(-(int)(signed char)(unsigned char)(k >> (8 * q)));
 #pragma unroll
-        for (int c = 0; c < VD; ++c) gr[c] = __half2float(__ushort_as_half(p[c])) * scale[grad_group<D>(c)];
+        for (int c = 0; c < VD; c += 8) {
+            const double2v d = chunk(c / 8);
+            unsigned short v[8];
+            __builtin_memcpy(v, &d, 16);
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (c + e < VD) gr[c + e] = __half2float(__ushort_as_half(v[e])) * scale[grad_group<D>(c + e)];
+        }
     }
 }
 
@@ -915,72 +927,111 @@ __global__ __launch_bounds__(CELL_BLOCK, LUNA_LANE_WAVES(L)) void k_sweep_lanes(
     block_min<CELL_BLOCK>(smallest, c.dt + (blockIdx.x % DT_SLOTS) * DT_STRIDE);
 }
 
-// finite_volume.hpp:1306-1329 FaceFlux::side() at order 1: half step (over step_dt) + g.r, positivity fallback. prow,
-// grow: the cell's primitive half and gradient row, read here so that only one side's rows are live at a time.
-template <int D>
-__device__ __forceinline__ void face_side(const Gas& gas, const double* prow, const double* grow, const double* off, double step_dt,
-                                          int order, double* Wf, int& fallbacks) {
+// One side of a face, from its cell's rows in memory. A gradient row of Prec: 16 B chunks GradientRow::CHUNKS.
+template <int D, int Prec>
+struct GradientRow {
+    static constexpr int CHUNKS = (Prec == 0 ? grad_row<D>() * 8 : Prec == 1 ? lp_row<D>() * 4 : HALF_ROW * 2) / 16;
+};
+template <int D, int Prec>
+struct MemorySide {
+    const double* row;
+    const double2v* grad;
+    __device__ __forceinline__ MemorySide(const Geo& g, const Rows& r, int i)
+        : row(g.cell + (size_t)i * CELL_ROW), grad(reinterpret_cast<const double2v*>(r.grad) + (size_t)i * GradientRow<D, Prec>::CHUNKS) {}
+    __device__ __forceinline__ void place(double* x, double* c) const {
+        using C = CellAt<D>;
+        load_vec<D>(row + C::X, x);
+        load_vec<D>(row + C::C, c);
+    }
+    __device__ __forceinline__ void state(double* W) const {
+#pragma unroll
+        for (int v = 0; v < D + 2; ++v) W[v] = row[CellAt<D>::W + v];
+    }
+    __device__ __forceinline__ double2v chunk(int k) const { return grad[k]; }
+};
+
+// The same from LDS, where a wavefront's 64 neighbours' rows are fetched in whole lines (as the sweep's Stage, whose reason
+// holds here: 14 loads a side of which each lane's touches a line of its own kept the L1's lookups at 85 % and the address
+// unit at 97 % of the flux kernel's time). The state part of a cell row is laid out as Stage does it; a gradient row keeps
+// its chunks together, chunk c of row l at place c ^ (l mod CHUNKS), so that lanes reading the same chunk of their rows
+// read different banks.
+template <int D, int Prec>
+struct StagedSide {
+    static constexpr int CELL = Stage<D>::CHUNKS, GRAD = GradientRow<D, Prec>::CHUNKS;
+    static constexpr int DOUBLES = 64 * 2 * (CELL + GRAD);
+    const lds_double* cell;
+    const lds_double* grad;
+    int lane;
+    __device__ __forceinline__ StagedSide(lds_double* lds, int lane) : cell(lds + lane * 2 * CELL), grad(lds + 64 * 2 * CELL + lane * 2 * GRAD), lane(lane) {}
+    // The rows of the cells j (one a lane; every lane of the wavefront active), asynchronously: finish() before reading.
+    static __device__ __forceinline__ void fetch(const Geo& g, const Rows& r, int j, bool gradients, lds_double* lds, int lane) {
+#pragma unroll
+        for (int k = 0; k < CELL; ++k) {
+            const int q = k * 64 + lane, c = q % CELL;
+            const unsigned of = (unsigned)__builtin_amdgcn_ds_bpermute(q / CELL * 4, j);
+            load(g.cell, (size_t)(of << 3 | (unsigned)(c < D ? c : c - D + GEO_ROW / 2)), lds + k * 128);
+        }
+        if (!gradients) return;
+#pragma unroll
+        for (int k = 0; k < GRAD; ++k) {
+            const int row = k * (64 / GRAD) + lane / GRAD;
+            const unsigned of = (unsigned)__builtin_amdgcn_ds_bpermute(row * 4, j);
+            load(r.grad, (size_t)of * GRAD + ((lane ^ row) & (GRAD - 1)), lds + 64 * 2 * CELL + k * 128);
+        }
+    }
+    static __device__ __forceinline__ void load(const double* from, size_t chunk, lds_double* to) {
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(reinterpret_cast<const char*>(from) + chunk * 16),
+                                         (__attribute__((address_space(3))) void*)to, 16, 0, 0);
+    }
+    static __device__ __forceinline__ void finish() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+    __device__ __forceinline__ void place(double* x, double* c) const {
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            x[a] = cell[a];
+            c[a] = cell[D + a];
+        }
+    }
+    __device__ __forceinline__ void state(double* W) const {
+#pragma unroll
+        for (int v = 0; v < D + 2; ++v) W[v] = cell[2 * D + v];
+    }
+    __device__ __forceinline__ double2v chunk(int k) const {
+        return *reinterpret_cast<const __attribute__((address_space(3))) double2v*>(grad + 2 * (k ^ (lane & (GRAD - 1))));
+    }
+};
+template <int D, class S>
+__device__ __forceinline__ void load_gradient(const S& side, double* gr) {
+#pragma unroll
+    for (int k = 0; k < (D + 2) * D; k += 2) {
+        const double2v d = side.chunk(k / 2);
+        gr[k] = d.x;
+        if (k + 1 < (D + 2) * D) gr[k + 1] = d.y;
+    }
+}
+
+// finite_volume.hpp:1306-1329 FaceFlux::side() at order 1: half step (over step_dt) + g.r, positivity fallback. The side's
+// rows are read here so that only one side's are live at a time. Reduced-precision policies (the float branch): W in double;
+// the gradient, the offset, the half step's rate and dt / 2 in float; W + (double)(g.r - dt/2 rate).
+template <int D, int Prec, class S>
+__device__ __forceinline__ void face_side(const Gas& gas, const Rows& r, int i, const S& side, const double* off, double step_dt, int order,
+                                          double* Wf, int& fallbacks) {
     constexpr int V = D + 2;
     double W[V];
-#pragma unroll
-    for (int v = 0; v < V; ++v) W[v] = prow[v];
+    side.state(W);
     if (order == 0) {
 #pragma unroll
         for (int v = 0; v < V; ++v) Wf[v] = W[v];
         return;
     }
-    double gr[V * D];
-#pragma unroll
-    for (int k = 0; k < V * D; ++k) gr[k] = grow[k];
-    half_step<D>(gas, W, gr, step_dt, Wf);
-#pragma unroll
-    for (int v = 0; v < V; ++v) Wf[v] += dot<D>(gr + v * D, off);
-    if (Wf[0] > 0 && Wf[D + 1] > 0) return;
-    ++fallbacks;
-#pragma unroll
-    for (int v = 0; v < V; ++v) Wf[v] = W[v];
-}
-
-// finite_volume.hpp:1451-1465 MovingFlux<false>::pass_side(): W + g.r on the mesh of t^n.
-template <int D>
-__device__ __forceinline__ void pass_side_first(const double* prow, const double* grow, const double* off, double* Wf, int& fallbacks) {
-    constexpr int V = D + 2;
-    double W[V];
-#pragma unroll
-    for (int v = 0; v < V; ++v) W[v] = prow[v];
-#pragma unroll
-    for (int v = 0; v < V; ++v) {
-        double gv[D];
-#pragma unroll
-        for (int a = 0; a < D; ++a) gv[a] = grow[v * D + a];
-        Wf[v] = W[v] + dot<D>(gv, off);
-    }
-    if (Wf[0] > 0 && Wf[D + 1] > 0) return;
-    ++fallbacks;
-#pragma unroll
-    for (int v = 0; v < V; ++v) Wf[v] = W[v];
-}
-
-// The sides of the reduced-precision policies (FaceFlux::side(), :1306-1329, float branch; MovingFlux<false>::pass_side(),
-// :1451-1465): W in double; the gradient, the offset, the half step's rate and dt / 2 in float; W + (double)(g.r - dt/2
-// rate) or W + (double)(g.r).
-template <int D, int Prec>
-__device__ __forceinline__ void face_side_p(const Gas& gas, const Rows& r, int i, const double* prow, const double* grow, const double* off,
-                                            double step_dt, int order, double* Wf, int& fallbacks) {
-    constexpr int V = D + 2;
     if constexpr (Prec == 0) {
-        face_side<D>(gas, prow, grow, off, step_dt, order, Wf, fallbacks);
+        double gr[V * D];
+        load_gradient<D>(side, gr);
+        half_step<D>(gas, W, gr, step_dt, Wf);
+#pragma unroll
+        for (int v = 0; v < V; ++v) Wf[v] += dot<D>(gr + v * D, off);
     } else {
-        double W[V];
-#pragma unroll
-        for (int v = 0; v < V; ++v) W[v] = prow[v];
-        if (order == 0) {
-#pragma unroll
-            for (int v = 0; v < V; ++v) Wf[v] = W[v];
-            return;
-        }
         float gr[V * D], Wg[V], A[V], rg[D];
-        load_gradient_lp<D, Prec>(r, i, gr);
+        decode_gradient<D, Prec>([&](int k) { return side.chunk(k); }, Prec == 2 ? r.exponents[i] : 0u, gr);
 #pragma unroll
         for (int v = 0; v < V; ++v) Wg[v] = (float)W[v];
         half_step_rate<D, float>(gas, Wg, gr, A);
@@ -989,105 +1040,94 @@ __device__ __forceinline__ void face_side_p(const Gas& gas, const Rows& r, int i
         const float h = 0.5f * (float)step_dt;
 #pragma unroll
         for (int v = 0; v < V; ++v) Wf[v] = W[v] + (double)(dot<D>(gr + v * D, rg) - h * A[v]);
-        if (Wf[0] > 0 && Wf[D + 1] > 0) return;
-        ++fallbacks;
-#pragma unroll
-        for (int v = 0; v < V; ++v) Wf[v] = W[v];
     }
-}
-template <int D, int Prec>
-__device__ __forceinline__ void pass_side_first_p(const Rows& r, int i, const double* prow, const double* grow, const double* off, double* Wf,
-                                                  int& fallbacks) {
-    constexpr int V = D + 2;
-    if constexpr (Prec == 0) {
-        pass_side_first<D>(prow, grow, off, Wf, fallbacks);
-    } else {
-        double W[V];
+    if (Wf[0] > 0 && Wf[D + 1] > 0) return;
+    ++fallbacks;
 #pragma unroll
-        for (int v = 0; v < V; ++v) W[v] = prow[v];
+    for (int v = 0; v < V; ++v) Wf[v] = W[v];
+}
+
+// finite_volume.hpp:1451-1465 MovingFlux<false>::pass_side(): W + g.r on the mesh of t^n (reduced precision: W + (double)(g.r)).
+template <int D, int Prec, class S>
+__device__ __forceinline__ void pass_side_first(const Rows& r, int i, const S& side, const double* off, double* Wf, int& fallbacks) {
+    constexpr int V = D + 2;
+    double W[V];
+    side.state(W);
+    if constexpr (Prec == 0) {
+        double gr[V * D];
+        load_gradient<D>(side, gr);
+#pragma unroll
+        for (int v = 0; v < V; ++v) Wf[v] = W[v] + dot<D>(gr + v * D, off);
+    } else {
         float gr[V * D], rg[D];
-        load_gradient_lp<D, Prec>(r, i, gr);
+        decode_gradient<D, Prec>([&](int k) { return side.chunk(k); }, Prec == 2 ? r.exponents[i] : 0u, gr);
 #pragma unroll
         for (int a = 0; a < D; ++a) rg[a] = (float)off[a];
 #pragma unroll
         for (int v = 0; v < V; ++v) Wf[v] = W[v] + (double)dot<D>(gr + v * D, rg);
-        if (Wf[0] > 0 && Wf[D + 1] > 0) return;
-        ++fallbacks;
-#pragma unroll
-        for (int v = 0; v < V; ++v) Wf[v] = W[v];
     }
-}
-
-// The position and centroid of one side of a face, and where its primitive half and gradient row are.
-template <int D>
-struct SideRows {
-    double x[D], c[D];
-    const double* p;
-    const double* g;
-};
-template <int D>
-__device__ __forceinline__ void load_side(const Geo& g, const Rows& r, int i, SideRows<D>& s) {
-    using C = CellAt<D>;
-    const double* row = g.cell + (size_t)i * CELL_ROW;
-    s.p = row + C::W;
-    s.g = r.grad + (size_t)i * grad_row<D>();
-    load_vec<D>(row + C::X, s.x);
-    load_vec<D>(row + C::C, s.c);
+    if (Wf[0] > 0 && Wf[D + 1] > 0) return;
+    ++fallbacks;
+#pragma unroll
+    for (int v = 0; v < V; ++v) Wf[v] = W[v];
 }
 
 __device__ __forceinline__ long long wrap_key(long long k, long long p);
 
+// A face as the flux reads it: A, the face centroid (relative to the owner's generator), owner, neighbour, |A|; from its 64 B
+// record (the per-cell loop, which gathers faces through the lists: one line each) or from the mesh's face arrays in place
+// (the per-face loop, which streams them).
+template <int D>
+struct Face {
+    double A[D], fc[D], magnitude;
+    int o, j;
+    __device__ __forceinline__ void from_record(const Geo& g, int f) {
+        using FA = FaceAt<D>;
+        const double* face = g.face + (size_t)f * FACE_ROW;
+        load_vec<D>(face + FA::A, A);
+        load_vec<D>(face + FA::FC, fc);
+        const int2 pair = *reinterpret_cast<const int2*>(face + FA::PAIR);
+        o = pair.x;
+        j = pair.y;
+        magnitude = face[FA::MAG];
+    }
+    __device__ __forceinline__ void from_arrays(const Geo& g, int f) {
+        load_vec<D>(g.area + (size_t)f * D, A);
+        load_vec<D>(g.fcen + (size_t)f * D, fc);
+        o = g.owner[f];
+        j = g.neighbour[f];
+        magnitude = sqrt(dot<D>(A, A));  // |A| as k_geo_faces writes it
+    }
+};
+
 // One face's flux times |A|: FaceFlux::operator() (:1415-1434) statically, MovingFlux::operator() (:1466-1490) on a moving
-// step; the positivity fallbacks of the owner's and the neighbour's side added to count_o and count_j. Record: read the
-// face from its 64 B record (the per-cell loop, which gathers faces through the lists: one line each), else from the
-// mesh's face arrays in place (the per-face loop, which streams them).
-template <int D, int Pass, int Riemann, int Prec, bool Record = false>
-__device__ __forceinline__ void flux_of_face(const Geo& g, const Rows& r, const Gas& gas, int order, double dt, double unit, int f, double* F,
-                                             int& count_o, int& count_j) {
+// step; the positivity fallbacks of the owner's and the neighbour's side added to count_o and count_j.
+template <int D, int Pass, int Riemann, int Prec, class SideO, class SideJ>
+__device__ __forceinline__ void flux_of_face(const Geo& g, const Rows& r, const Gas& gas, int order, double dt, double unit, const Face<D>& face,
+                                             const SideO& so, const SideJ& sj, double* F, int& count_o, int& count_j) {
     constexpr int V = D + 2;
-    using FA = FaceAt<D>;
     {
-        // A, the face centroid (relative to the owner's generator), owner, neighbour, |A|
-        double rec[FACE_ROW - 1];
-        int o, j;
-        double magnitude;
-        if constexpr (Record) {
-            const double* face = g.face + (size_t)f * FACE_ROW;
-#pragma unroll
-            for (int k = 0; k < FACE_ROW - 1; ++k) rec[k] = face[k];
-            const int2 pair = *reinterpret_cast<const int2*>(face + FA::PAIR);
-            o = pair.x;
-            j = pair.y;
-            magnitude = rec[FA::MAG];
-        } else {
-#pragma unroll
-            for (int k = 0; k < D; ++k) {
-                rec[FA::A + k] = g.area[(size_t)f * D + k];
-                rec[FA::FC + k] = g.fcen[(size_t)f * D + k];
-            }
-            o = g.owner[f];
-            j = g.neighbour[f];
-            magnitude = sqrt(dot<D>(rec + FA::A, rec + FA::A));  // |A| as k_geo_faces writes it
-        }
+        const int o = face.o, j = face.j;
+        const double magnitude = face.magnitude;
 #pragma unroll
         for (int v = 0; v < V; ++v) F[v] = 0;
         if (magnitude != 0) {
-            SideRows<D> so, sj;
-            load_side<D>(g, r, o, so);
-            load_side<D>(g, r, j, sj);
+            double xo[D], xj[D], co[D], cj[D];
+            so.place(xo, co);
+            sj.place(xj, cj);
             double L[V], R[V], n[D], wf[D], ro[D], rj[D], d[D];
             const double inv = 1.0 / magnitude;
 #pragma unroll
             for (int k = 0; k < D; ++k) {
-                n[k] = rec[FA::A + k] * inv;
+                n[k] = face.A[k] * inv;
                 wf[k] = 0;
             }
             // face_offset (:322-326) of both sides
-            separation<D>(g, sj.x, so.x, d);  // the owner seen from the neighbour
+            separation<D>(g, xj, xo, d);  // the owner seen from the neighbour
 #pragma unroll
             for (int k = 0; k < D; ++k) {
-                ro[k] = rec[FA::FC + k] - so.c[k];
-                rj[k] = rec[FA::FC + k] + d[k] - sj.c[k];
+                ro[k] = face.fc[k] - co[k];
+                rj[k] = face.fc[k] + d[k] - cj[k];
             }
             if constexpr (Pass < 0) {
                 const double half = 0.5 * dt;
@@ -1096,8 +1136,8 @@ __device__ __forceinline__ void flux_of_face(const Geo& g, const Rows& r, const 
                     ro[k] = ro[k] + wf[k] * half;
                     rj[k] = rj[k] + wf[k] * half;
                 }
-                face_side_p<D, Prec>(gas, r, o, so.p, so.g, ro, dt, order, L, count_o);
-                face_side_p<D, Prec>(gas, r, j, sj.p, sj.g, rj, dt, order, R, count_j);
+                face_side<D, Prec>(gas, r, o, so, ro, dt, order, L, count_o);
+                face_side<D, Prec>(gas, r, j, sj, rj, dt, order, R, count_j);
             } else {
                 double wo[D], wj[D];
 #pragma unroll
@@ -1112,11 +1152,11 @@ __device__ __forceinline__ void flux_of_face(const Geo& g, const Rows& r, const 
                 }
                 // face_velocity (:1380-1397)
                 double sep[D], cf[D], dw[D];
-                separation<D>(g, so.x, sj.x, sep);
+                separation<D>(g, xo, xj, sep);
                 const double dist = sqrt(dot<D>(sep, sep));
                 const double inv_dist = 1.0 / dist;
 #pragma unroll
-                for (int k = 0; k < D; ++k) cf[k] = rec[FA::FC + k] - sep[k] * 0.5;
+                for (int k = 0; k < D; ++k) cf[k] = face.fc[k] - sep[k] * 0.5;
 #pragma unroll
                 for (int k = 0; k < D; ++k) dw[k] = wo[k] - wj[k];
                 double facv = dot<D>(cf, dw) * inv_dist;
@@ -1125,11 +1165,11 @@ __device__ __forceinline__ void flux_of_face(const Geo& g, const Rows& r, const 
 #pragma unroll
                 for (int k = 0; k < D; ++k) wf[k] = (wo[k] + wj[k]) * 0.5 + sep[k] * (facv * inv_dist);
                 if constexpr (Pass == 2) {
-                    face_side_p<D, Prec>(gas, r, o, so.p, so.g, ro, dt, 0, L, count_o);
-                    face_side_p<D, Prec>(gas, r, j, sj.p, sj.g, rj, dt, 0, R, count_j);
+                    face_side<D, Prec>(gas, r, o, so, ro, dt, 0, L, count_o);
+                    face_side<D, Prec>(gas, r, j, sj, rj, dt, 0, R, count_j);
                 } else if constexpr (Pass == 0) {
-                    pass_side_first_p<D, Prec>(r, o, so.p, so.g, ro, L, count_o);
-                    pass_side_first_p<D, Prec>(r, j, sj.p, sj.g, rj, R, count_j);
+                    pass_side_first<D, Prec>(r, o, so, ro, L, count_o);
+                    pass_side_first<D, Prec>(r, j, sj, rj, R, count_j);
                 } else {
                     // side(i, r + c^n+1 - c^n + w dt) with the FaceFlux dt = 2 dt (:1452-1454)
                     const double step_dt = 2 * dt;
@@ -1137,15 +1177,15 @@ __device__ __forceinline__ void flux_of_face(const Geo& g, const Rows& r, const 
 #pragma unroll
                     for (int k = 0; k < D; ++k) {
                         const double moved = wo[k] * (0.5 * step_dt);
-                        r2[k] = ro[k] + so.c[k] - r.old_centroid[(size_t)o * D + k] + moved;
+                        r2[k] = ro[k] + co[k] - r.old_centroid[(size_t)o * D + k] + moved;
                     }
-                    face_side_p<D, Prec>(gas, r, o, so.p, so.g, r2, step_dt, 1, L, count_o);
+                    face_side<D, Prec>(gas, r, o, so, r2, step_dt, 1, L, count_o);
 #pragma unroll
                     for (int k = 0; k < D; ++k) {
                         const double moved = wj[k] * (0.5 * step_dt);
-                        r2[k] = rj[k] + sj.c[k] - r.old_centroid[(size_t)j * D + k] + moved;
+                        r2[k] = rj[k] + cj[k] - r.old_centroid[(size_t)j * D + k] + moved;
                     }
-                    face_side_p<D, Prec>(gas, r, j, sj.p, sj.g, r2, step_dt, 1, R, count_j);
+                    face_side<D, Prec>(gas, r, j, sj, r2, step_dt, 1, R, count_j);
                 }
             }
             if constexpr (Riemann == 1)
@@ -1163,21 +1203,34 @@ __device__ __forceinline__ void flux_of_face(const Geo& g, const Rows& r, const 
     }
 }
 
-// One face's flux row per work-item (the per-face loop, Update::per_face).
+// One face's flux row per work-item (the per-face loop, Update::per_face), one wavefront per work-group. The owner's rows are
+// read in place (faces come in runs of one owner), the neighbour's through LDS. With both sides' rows loaded lane by lane the
+// address unit was busy 97 % of the time; now 11 wavefronts a CU (14 KiB of LDS each) wait for their rows: 128^3 static 0.71
+// -> 0.59 ms, 104^3 moving passes 0.42 -> 0.36 and 0.48 -> 0.42, FP16 rows at 72^3 0.106 -> 0.097.
 template <int D, int Pass, int Riemann, int Prec = 0>
-__global__ __launch_bounds__(BLOCK, LUNA_FLUX_WAVES) void k_flux(Geo g, Rows r, Gas gas, int order, double dt, double unit, unsigned long long* fallbacks) {
+__global__ __launch_bounds__(CELL_BLOCK, LUNA_FLUX_WAVES) void k_flux(Geo g, Rows r, Gas gas, int order, double dt, double unit, unsigned long long* fallbacks) {
     constexpr int V = D + 2;
-    const int f = xcd_block() * BLOCK + threadIdx.x;
+    using Staged = StagedSide<D, Prec>;
+    __shared__ double rows[Staged::DOUBLES];
+    lds_double* lds = (lds_double*)rows;
+    const int lane = threadIdx.x, f = xcd_block() * CELL_BLOCK + lane;
     int count = 0;
-    if (f < g.F) {
-        double F[V];
-        int co = 0, cj = 0;
-        flux_of_face<D, Pass, Riemann, Prec>(g, r, gas, order, dt, unit, f, F, co, cj);
-        count = co + cj;
+    if (g.F > 0) {
+        const int at = min(f, g.F - 1);
+        Staged::fetch(g, r, g.neighbour[at], Pass != 2 && order != 0, lds, lane);
+        Face<D> face;
+        face.from_arrays(g, at);
+        Staged::finish();
+        if (f < g.F) {
+            double F[V];
+            int co = 0, cj = 0;
+            flux_of_face<D, Pass, Riemann, Prec>(g, r, gas, order, dt, unit, face, MemorySide<D, Prec>(g, r, face.o), Staged(lds, lane), F, co, cj);
+            count = co + cj;
 #pragma unroll
-        for (int v = 0; v < V; ++v) r.flux[(size_t)f * V + v] = F[v];
+            for (int v = 0; v < V; ++v) r.flux[(size_t)f * V + v] = F[v];
+        }
     }
-    block_count<BLOCK>(count, fallbacks);
+    block_count<CELL_BLOCK>(count, fallbacks);
 }
 
 // finite_volume.hpp:1544-1566 fluxes_and_update (Update::per_cell): each cell computes the flux of every face in its list
@@ -1199,7 +1252,10 @@ __global__ __launch_bounds__(CELL_BLOCK) void k_fluxes_and_update(Geo g, Rows r,
             const int e = g.list[base + t * SLICE], f = e >= 0 ? e : ~e;
             double F[V];
             int co = 0, cj = 0;
-            flux_of_face<D, Pass, Riemann, Prec, true>(g, r, gas, order, flux_dt, unit, f, F, co, cj);
+            Face<D> face;
+            face.from_record(g, f);
+            flux_of_face<D, Pass, Riemann, Prec>(g, r, gas, order, flux_dt, unit, face, MemorySide<D, Prec>(g, r, face.o),
+                                                 MemorySide<D, Prec>(g, r, face.j), F, co, cj);
             count += e >= 0 ? co : cj;
             const double sign = e >= 0 ? 1.0 : -1.0;
 #pragma unroll
@@ -1391,13 +1447,13 @@ hipError_t launch_sweep(hipStream_t s, const Geo& g, const Rows& r, const Gas& g
 template <int D, int Pass, int Prec>
 static hipError_t flux_prec(hipStream_t s, const Geo& g, const Rows& r, const Gas& gas, int riemann, int order, double dt, double unit,
                             unsigned long long* fallbacks) {
-    const dim3 grid = blocks(g.F > 0 ? g.F : 1);
+    const dim3 grid = blocks(g.F > 0 ? g.F : 1, CELL_BLOCK);
     if (riemann == 1)
-        hipLaunchKernelGGL((k_flux<D, Pass, 1, Prec>), grid, dim3(BLOCK), 0, s, g, r, gas, order, dt, unit, fallbacks);
+        hipLaunchKernelGGL((k_flux<D, Pass, 1, Prec>), grid, dim3(CELL_BLOCK), 0, s, g, r, gas, order, dt, unit, fallbacks);
     else if (Prec == 0 && riemann == 2)
-        hipLaunchKernelGGL((k_flux<D, Pass, 2, 0>), grid, dim3(BLOCK), 0, s, g, r, gas, order, dt, unit, fallbacks);
+        hipLaunchKernelGGL((k_flux<D, Pass, 2, 0>), grid, dim3(CELL_BLOCK), 0, s, g, r, gas, order, dt, unit, fallbacks);
     else
-        hipLaunchKernelGGL((k_flux<D, Pass, 0, Prec>), grid, dim3(BLOCK), 0, s, g, r, gas, order, dt, unit, fallbacks);
+        hipLaunchKernelGGL((k_flux<D, Pass, 0, Prec>), grid, dim3(CELL_BLOCK), 0, s, g, r, gas, order, dt, unit, fallbacks);
     return hipGetLastError();
 }
 template <int D, int Pass>
