@@ -3,6 +3,8 @@
 // runs in list order, one work-item per cell, and every face's share is computed by one work-item per face, so the
 // results are deterministic (no atomics) and follow the CPU restatement's operation order. The forward pieces (fit,
 // limiter, face sides) are recomputed with the forward's own arithmetic.
+#include <type_traits>
+
 #include "derivatives.hpp"
 #include "kernels.hpp"
 
@@ -42,55 +44,82 @@ __device__ __forceinline__ void separation(const Geo& g, const double* xi, const
     for (int a = 0; a < D; ++a) d[a] = wrap(xj[a] - xi[a], g.side[a], g.inverse[a]);
 }
 
-// Geometry::face_offset (finite_volume.hpp:322-326) of face f from cell i (fc is stored relative to the owner).
+// Geometry::face_offset (finite_volume.hpp:322-326): the face centroid relative to the cell's centroid, kept per slot.
 template <int D>
-__device__ __forceinline__ void face_offset(const Geo& g, const double* face, bool owned, const double* xi, const double* ci, int other,
-                                            double* r) {
-    using C = CellAt<D>;
-    double rel[D];
-    load_vec<D>(face + FaceAt<D>::FC, rel);
-    if (!owned) {
-        double xo[D], s[D];
-        load_vec<D>(g.cell + (size_t)other * CELL_ROW + C::X, xo);
-        separation<D>(g, xi, xo, s);
+__device__ __forceinline__ void face_offset(const Geo& g, int slot, double* r) {
 #pragma unroll
-        for (int a = 0; a < D; ++a) rel[a] = rel[a] + s[a];
-    }
-#pragma unroll
-    for (int a = 0; a < D; ++a) r[a] = rel[a] - ci[a];
+    for (int a = 0; a < D; ++a) r[a] = g.slot[(a + 1) * g.slots + slot];
 }
 
 // What the face-centroid limiter did per variable (finite_volume.hpp:709-799): the last clipping face (list position, -1
-// none), its offset, the bound and the face whose neighbour holds it (the first entry in list order with the extreme).
+// none), whether it took the upper bound and zeroed the slope, the bound and the list entry whose neighbour holds it (the
+// first in list order with the extreme). The clipping face's offset and the bound's tangent are read again where they are
+// needed (face_offset, bound_tangent): carried through the walks they cost 50 registers.
 template <int D>
 struct Pattern {
     int last[D + 2], extreme[D + 2];
     bool upper[D + 2], zero[D + 2];
-    double offset[D + 2][D], bound[D + 2], dbound[D + 2];
+    double bound[D + 2];
 };
+template <int D>
+__device__ __forceinline__ double bound_tangent(const Geo& g, int base, const Pattern<D>& pat, int v, const double* dW) {
+    return pat.extreme[v] < 0 ? 0.0 : dW[(size_t)g.other[base + pat.extreme[v] * SLICE] * (D + 2) + v];
+}
+
+// M x = b of the fit with its Cholesky factor L, in the sweep's operation order. Fast: with the correctly rounded quotients of
+// exact_math.hpp by L's diagonal (by), the same bits for operands in their range.
+template <int D, bool Fast>
+__device__ __forceinline__ void solve_fit(const double (*L)[D + 1], const Divisor* by, const double* b, double* x) {
+    constexpr int U = D + 1;
+    double z[U];
+#pragma unroll
+    for (int p = 0; p < U; ++p) {
+        double sum = b[p];
+#pragma unroll
+        for (int m = 0; m < p; ++m) sum -= L[p][m] * z[m];
+        z[p] = Fast ? over(sum, by[p]) : sum / L[p][p];
+    }
+#pragma unroll
+    for (int p = U - 1; p >= 0; --p) {
+        double sum = z[p];
+#pragma unroll
+        for (int m = p + 1; m < U; ++m) sum -= L[m][p] * x[m];
+        x[p] = Fast ? over(sum, by[p]) : sum / L[p][p];
+    }
+}
+// Whether solves with this factor and right-hand sides of absolute sum `size` stay in the fast quotients' range: diagonals
+// within 2^200 of 1 and a size under 2^200 bound every quotient on the way by 2^1000.
+template <int D>
+__device__ __forceinline__ bool solves_fast(const double (*L)[D + 1], double size) {
+    bool ok = size < 0x1p200;
+#pragma unroll
+    for (int p = 0; p <= D; ++p) ok = ok && L[p][p] > 0x1p-200 && L[p][p] < 0x1p200;
+    return ok;
+}
 
 // The cell's fit and limiter as the sweep computes them (the same bits for g), with the unlimited gradient g0, its tangent
-// dg0 (Tangent), M's Cholesky factor L and first row M0, and the limiter's pattern. dW: N x V tangents of W.
+// dg0 (Tangent), M's Cholesky factor L and first row M0, and the limiter's pattern. dW: N x V tangents of W. The walks read
+// |A| and the face offsets from the slots; the surface is summed first, so that the range leaves out the tiny faces as it
+// goes (a second walk for them ran in nearly every wavefront). With 64 B face records gathered twice an entry, that second
+// walk and the compiler's 46 divisions a solve the fit's tangent took 0.55 ms at 80^3 and the cell adjoint 0.34 at 56^3; now
+// 0.35 and 0.21, without spills.
 template <int D, bool Tangent>
 __device__ void fit_cell(const Geo& g, int i, const double* dW, bool limit, double* gl, double* g0, double* dg0, double (*L)[D + 1],
                          double* M0, Pattern<D>& pat, double* intercept = nullptr) {
     constexpr int V = D + 2, U = D + 1;
     using C = CellAt<D>;
-    using FA = FaceAt<D>;
     const double* mine = g.cell + (size_t)i * CELL_ROW;
     double Wi[V], xi[D], ci[D];
 #pragma unroll
     for (int v = 0; v < V; ++v) Wi[v] = mine[C::W + v];
     load_vec<D>(mine + C::X, xi);
     load_vec<D>(mine + C::C, ci);
-    double surface = 0, smallest = INFINITY;
-    double lo[V], hi[V], dlo[V], dhi[V];
+    double lo[V], hi[V];
     int lo_f[V], hi_f[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) {
         lo[v] = 1.7976931348623157e308;
         hi[v] = -1.7976931348623157e308;
-        dlo[v] = dhi[v] = 0;
         lo_f[v] = hi_f[v] = -1;
     }
     double M[U][U], b[V][U], db[V][U];
@@ -103,18 +132,30 @@ __device__ void fit_cell(const Geo& g, int i, const double* dW, bool limit, doub
 #pragma unroll
         for (int p = 0; p < U; ++p) b[v][p] = db[v][p] = 0;
     const int count = g.count[i], base = first_slot(g, i);
+    double surface = 0;
+    for (int k = 0; k < count; k += 4) {
+        double m[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) m[u] = g.slot[base + min(k + u, count - 1) * SLICE];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (k + u < count) surface += m[u];
+    }
+    const double tiny = 1e-6 * surface;
+    int next = count > 0 ? g.other[base] : 0;
     for (int k = 0; k < count; ++k) {
-        const int slot = base + k * SLICE;
-        const int e = g.list[slot], f = e >= 0 ? e : ~e, j = g.other[slot];
+        const int slot = base + k * SLICE, j = next;
+        next = g.other[base + min(k + 1, count - 1) * SLICE];
         const double* row = g.cell + (size_t)j * CELL_ROW;
-        double xj[D], d[D], X[U], Wj[V];
+        double xj[D], d[D], X[U], Wj[V], dWj[V];
         load_vec<D>(row + C::X, xj);
         separation<D>(g, xi, xj, d);
 #pragma unroll
-        for (int v = 0; v < V; ++v) Wj[v] = row[C::W + v];
-        const double w = g.face[(size_t)f * FACE_ROW + FA::MAG];
-        surface += w;
-        smallest = fmin(smallest, w);
+        for (int v = 0; v < V; ++v) {
+            Wj[v] = row[C::W + v];
+            if constexpr (Tangent) dWj[v] = dW[(size_t)j * V + v];
+        }
+        const double w = g.slot[slot];
         X[0] = 1;
 #pragma unroll
         for (int p = 1; p < U; ++p) X[p] = d[p - 1] + row[C::C + p - 1] - ci[p - 1];
@@ -127,36 +168,17 @@ __device__ void fit_cell(const Geo& g, int i, const double* dW, bool limit, doub
             const double dWv = Wj[v] - Wi[v];
 #pragma unroll
             for (int p = 0; p < U; ++p) b[v][p] += w * X[p] * dWv;
-            double dWj = 0;
             if constexpr (Tangent) {
-                dWj = dW[(size_t)j * V + v];
-                const double ddW = w * (dWj - dW[(size_t)i * V + v]);
+                const double ddW = w * (dWj[v] - dW[(size_t)i * V + v]);
 #pragma unroll
                 for (int p = 0; p < U; ++p) db[v][p] += X[p] * ddW;
             }
-            if (Wj[v] < lo[v]) lo[v] = Wj[v], lo_f[v] = k, dlo[v] = dWj;
-            if (Wj[v] > hi[v]) hi[v] = Wj[v], hi_f[v] = k, dhi[v] = dWj;
         }
-    }
-    const double tiny = 1e-6 * surface;
-    const bool any_tiny = smallest < tiny;
-    if (any_tiny) {
-#pragma unroll
-        for (int v = 0; v < V; ++v) {
-            lo[v] = 1.7976931348623157e308;
-            hi[v] = -1.7976931348623157e308;
-            lo_f[v] = hi_f[v] = -1;
-        }
-        for (int k = 0; k < count; ++k) {
-            const int slot = base + k * SLICE;
-            const int e = g.list[slot], f = e >= 0 ? e : ~e, j = g.other[slot];
-            if (g.face[(size_t)f * FACE_ROW + FA::MAG] < tiny) continue;
-            const double* row = g.cell + (size_t)j * CELL_ROW + C::W;
+        if (!(w < tiny)) {
 #pragma unroll
             for (int v = 0; v < V; ++v) {
-                const double dWj = Tangent ? dW[(size_t)j * V + v] : 0.0;
-                if (row[v] < lo[v]) lo[v] = row[v], lo_f[v] = k, dlo[v] = dWj;
-                if (row[v] > hi[v]) hi[v] = row[v], hi_f[v] = k, dhi[v] = dWj;
+                if (Wj[v] < lo[v]) lo[v] = Wj[v], lo_f[v] = k;
+                if (Wj[v] > hi[v]) hi[v] = Wj[v], hi_f[v] = k;
             }
         }
     }
@@ -174,76 +196,69 @@ __device__ void fit_cell(const Geo& g, int i, const double* dW, bool limit, doub
             for (int m = 0; m < q; ++m) sum -= L[p][m] * L[q][m];
             L[p][q] = p == q ? sqrt(sum) : sum / L[q][q];
         }
+    double size = 0;
 #pragma unroll
     for (int p = 0; p < U; ++p) M0[p] = M[0][p];
 #pragma unroll
-    for (int pass = 0; pass < (Tangent ? 2 : 1); ++pass) {
+    for (int v = 0; v < V; ++v)
+#pragma unroll
+        for (int p = 0; p < U; ++p) size += fabs(b[v][p]) + (Tangent ? fabs(db[v][p]) : 0.0);
+    const auto solve = [&](auto fast) {
+        constexpr bool Fast = decltype(fast)::value;
+        Divisor by[U];
+#pragma unroll
+        for (int p = 0; p < U; ++p) by[p] = Fast ? divisor(L[p][p]) : Divisor{L[p][p], 0.0};
 #pragma unroll
         for (int v = 0; v < V; ++v) {
-            double z[U], x[U];
+            double x[U];
+            solve_fit<D, Fast>(L, by, b[v], x);
 #pragma unroll
-            for (int p = 0; p < U; ++p) {
-                double sum = pass == 0 ? b[v][p] : db[v][p];
+            for (int a = 0; a < D; ++a) g0[v * D + a] = gl[v * D + a] = x[1 + a];
+            if (intercept) intercept[v] = x[0];
+            if constexpr (Tangent) {
+                solve_fit<D, Fast>(L, by, db[v], x);
 #pragma unroll
-                for (int m = 0; m < p; ++m) sum -= L[p][m] * z[m];
-                z[p] = sum / L[p][p];
+                for (int a = 0; a < D; ++a) dg0[v * D + a] = x[1 + a];
             }
-#pragma unroll
-            for (int p = U - 1; p >= 0; --p) {
-                double sum = z[p];
-#pragma unroll
-                for (int m = p + 1; m < U; ++m) sum -= L[m][p] * x[m];
-                x[p] = sum / L[p][p];
-            }
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-                if (pass == 0)
-                    g0[v * D + a] = gl[v * D + a] = x[1 + a];
-                else
-                    dg0[v * D + a] = x[1 + a];
-            }
-            if (pass == 0 && intercept) intercept[v] = x[0];
         }
-    }
+    };
+    if (__all(solves_fast<D>(L, size)))
+        solve(std::true_type{});
+    else
+        solve(std::false_type{});
 #pragma unroll
     for (int v = 0; v < V; ++v) {
-        pat.last[v] = pat.extreme[v] = -1;
-        pat.upper[v] = pat.zero[v] = false;
+        pat.last[v] = -1;
+        pat.upper[v] = false;
     }
     if (limit)
         for (int k = 0; k < count; ++k) {
             const int slot = base + k * SLICE;
-            const int e = g.list[slot], f = e >= 0 ? e : ~e;
-            const double* face = g.face + (size_t)f * FACE_ROW;
-            if (any_tiny && face[FA::MAG] < tiny) continue;
             double offset[D];
-            face_offset<D>(g, face, e >= 0, xi, ci, g.other[slot], offset);
+            face_offset<D>(g, slot, offset);
+            if (g.slot[slot] < tiny) continue;
+            double dp[V];
+            bool up[V], down[V];
 #pragma unroll
             for (int v = 0; v < V; ++v) {
-                double* gv = gl + v * D;
-                const double dp = dot<D>(gv, offset);
-                if (dp > 0 && Wi[v] + dp > hi[v]) {
-                    const double s = hi[v] > Wi[v] ? (hi[v] - Wi[v]) / dp : 0.0;
+                dp[v] = dot<D>(gl + v * D, offset);
+                up[v] = dp[v] > 0 && Wi[v] + dp[v] > hi[v];
+                down[v] = dp[v] < 0 && Wi[v] + dp[v] < lo[v];
+            }
 #pragma unroll
-                    for (int a = 0; a < D; ++a) gv[a] = gv[a] * s;
-                    pat.last[v] = k, pat.upper[v] = true, pat.zero[v] = !(hi[v] > Wi[v]);
+            for (int v = 0; v < V; ++v) {
+                if (!(up[v] || down[v])) continue;
+                const double room = (up[v] ? hi[v] : lo[v]) - Wi[v], q = room / dp[v], s = q > 0 ? q : 0.0;
 #pragma unroll
-                    for (int a = 0; a < D; ++a) pat.offset[v][a] = offset[a];
-                } else if (dp < 0 && Wi[v] + dp < lo[v]) {
-                    const double s = lo[v] < Wi[v] ? (lo[v] - Wi[v]) / dp : 0.0;
-#pragma unroll
-                    for (int a = 0; a < D; ++a) gv[a] = gv[a] * s;
-                    pat.last[v] = k, pat.upper[v] = false, pat.zero[v] = !(lo[v] < Wi[v]);
-#pragma unroll
-                    for (int a = 0; a < D; ++a) pat.offset[v][a] = offset[a];
-                }
+                for (int a = 0; a < D; ++a) gl[v * D + a] = gl[v * D + a] * s;
+                pat.last[v] = k, pat.upper[v] = up[v];
             }
         }
 #pragma unroll
     for (int v = 0; v < V; ++v) {
         pat.extreme[v] = pat.last[v] < 0 ? -1 : pat.upper[v] ? hi_f[v] : lo_f[v];
         pat.bound[v] = pat.upper[v] ? hi[v] : lo[v];
-        pat.dbound[v] = pat.upper[v] ? dhi[v] : dlo[v];
+        pat.zero[v] = pat.last[v] >= 0 && (pat.upper[v] ? !(hi[v] > Wi[v]) : !(lo[v] < Wi[v]));
     }
 }
 
@@ -348,6 +363,7 @@ __global__ __launch_bounds__(BLOCK, LUNA_DERIV_WAVES) void k_fit_tangent(Geo g, 
     double gl[V * D], g0[V * D], dg0[V * D], L[U][U], M0[U];
     Pattern<D> pat;
     fit_cell<D, true>(g, i, dW, limit != 0, gl, g0, dg0, L, M0, pat);
+    const int base = first_slot(g, i);
     const double* Wi = g.cell + (size_t)i * CELL_ROW + C::W;
     const double* dWi = dW + (size_t)i * V;
     double* out = r.grad + (size_t)i * GR;
@@ -365,9 +381,10 @@ __global__ __launch_bounds__(BLOCK, LUNA_DERIV_WAVES) void k_fit_tangent(Geo g, 
 #pragma unroll
             for (int a = 0; a < D; ++a) dout[v * D + a] = 0.0;
         } else {
-            const double* o = pat.offset[v];
+            double o[D];
+            face_offset<D>(g, base + pat.last[v] * SLICE, o);
             const double den = dot<D>(gv, o);
-            const double s = (pat.bound[v] - Wi[v]) / den, ds = (pat.dbound[v] - dWi[v] - s * dot<D>(dgv, o)) / den;
+            const double s = (pat.bound[v] - Wi[v]) / den, ds = (bound_tangent<D>(g, base, pat, v, dW) - dWi[v] - s * dot<D>(dgv, o)) / den;
 #pragma unroll
             for (int a = 0; a < D; ++a) dout[v * D + a] = dgv[a] * s + gv[a] * ds;
         }
@@ -539,35 +556,17 @@ __global__ __launch_bounds__(BLOCK, LUNA_DERIV_WAVES) void k_cell_adjoint(Geo g,
     // This cell's side of each of its faces, as face_sides computes it for the face kernel: the half step is the cell's
     // own (the same for all its faces), plus g . r with r the face centroid in this cell's frame minus its centroid; only
     // the fallback flag and r are needed here, so the other side's rows are not read.
-    double hs[V], ci[D], xi[D];
+    double hs[V];
     half_step<D>(gas, Wi, gi, dt, hs);
-    load_vec<D>(g.cell + (size_t)i * CELL_ROW + C::C, ci);
-    load_vec<D>(g.cell + (size_t)i * CELL_ROW + C::X, xi);
     const double half = 0.5 * dt, wf = 0.0;
     const int count = g.count[i], base = first_slot(g, i);
     for (int k = 0; k < count; ++k) {
-        const int e = g.list[base + k * SLICE], f = e >= 0 ? e : ~e;
-        const double* face = g.face + (size_t)f * FACE_ROW;
-        if (face[FaceAt<D>::MAG] == 0) continue;
-        const int s = e >= 0 ? 0 : 1;
+        const int slot = base + k * SLICE, e = g.list[slot], f = e >= 0 ? e : ~e, s = e >= 0 ? 0 : 1;
+        if (g.slot[slot] == 0) continue;
         double rr[D];
-        if (s == 0) {
+        face_offset<D>(g, slot, rr);
 #pragma unroll
-            for (int c = 0; c < D; ++c) {
-                rr[c] = face[FaceAt<D>::FC + c] - ci[c];
-                rr[c] = rr[c] + wf * half;
-            }
-        } else {
-            const int2 pair = *reinterpret_cast<const int2*>(face + FaceAt<D>::PAIR);
-            double xo[D], d[D];
-            load_vec<D>(g.cell + (size_t)pair.x * CELL_ROW + C::X, xo);
-            separation<D>(g, xi, xo, d);  // the owner seen from this cell, the neighbour
-#pragma unroll
-            for (int c = 0; c < D; ++c) {
-                rr[c] = face[FaceAt<D>::FC + c] + d[c] - ci[c];
-                rr[c] = rr[c] + wf * half;
-            }
-        }
+        for (int c = 0; c < D; ++c) rr[c] = rr[c] + wf * half;
         double Wf[V];
 #pragma unroll
         for (int v = 0; v < V; ++v) Wf[v] = hs[v] + dot<D>(gi + v * D, rr);
@@ -605,7 +604,8 @@ __global__ __launch_bounds__(BLOCK, LUNA_DERIV_WAVES) void k_cell_adjoint(Geo g,
 #pragma unroll
             for (int c = 0; c < D; ++c) g0bar[c] = 0;
         } else if (pat.last[v] >= 0) {
-            const double* o = pat.offset[v];
+            double o[D];
+            face_offset<D>(g, base + pat.last[v] * SLICE, o);
             const double den = dot<D>(g0 + v * D, o);
             const double sc = (pat.bound[v] - Wi[v]) / den;
             t = dot<D>(gb + v * D, g0 + v * D) / den;
@@ -1146,7 +1146,8 @@ __global__ __launch_bounds__(BLOCK) void k_mcell_adjoint(Geo g, Rows r, Gas gas,
 #pragma unroll
             for (int a = 0; a < D; ++a) g0bar[a] = 0;
         } else if (pat.last[v] >= 0) {
-            const double* o = pat.offset[v];
+            double o[D];
+            face_offset<D>(g, base + pat.last[v] * SLICE, o);
             const double den = dot<D>(g0 + v * D, o);
             const double sc = (pat.bound[v] - Wi[v]) / den;
             t = dot<D>(gb + v * D, g0 + v * D) / den;
@@ -1622,13 +1623,14 @@ __global__ __launch_bounds__(BLOCK) void k_mcell_tangent(Geo g, Rows r, int limi
             const int e = g.list[slot], f = e >= 0 ? e : ~e;
             double dor[D];
             offset_dot<D>(dxf + (size_t)f * D, e >= 0, dxi, dx + (size_t)g.other[slot] * D, dci, dor);
-            const double* o = pat.offset[v];
+            double o[D];
+            face_offset<D>(g, base + pat.last[v] * SLICE, o);
             double dg0v[D];
 #pragma unroll
             for (int a = 0; a < D; ++a) dg0v[a] = xs[1 + a];
             const double den = dot<D>(gv, o);
             const double sc = (pat.bound[v] - Wi[v]) / den;
-            const double dsc = (pat.dbound[v] - dWi[v] - sc * (dot<D>(dg0v, o) + dot<D>(gv, dor))) / den;
+            const double dsc = (bound_tangent<D>(g, base, pat, v, dW) - dWi[v] - sc * (dot<D>(dg0v, o) + dot<D>(gv, dor))) / den;
 #pragma unroll
             for (int a = 0; a < D; ++a) out[v * D + a] = dg0v[a] * sc + gv[a] * dsc;
         }
