@@ -5,6 +5,7 @@
 #include <climits>
 #include <cmath>
 #include <algorithm>
+#include <chrono>
 #include <cstdio>
 #include <thread>
 #include <cstring>
@@ -220,7 +221,7 @@ struct luna_fv {
     int riemann() const {
         return opt.hll_compression > 0 && opt.riemann == LUNA_RIEMANN_HLLC ? 2 : opt.riemann;
     }
-    luna::Gas gas() const { return luna::Gas{opt.gamma, opt.smallr, opt.smallc, 1.0 / (opt.gamma - 1.0)}; }
+    luna::Gas gas() const { return luna::make_gas(opt.gamma, opt.smallr, opt.smallc); }
     luna::Counters counters_now() const {
         return luna::Counters{counters.p + parity * luna::DT_WORDS, counters.p + (parity ^ 1) * luna::DT_WORDS, fallback_counters()};
     }
@@ -1425,7 +1426,7 @@ struct luna_fv1 {
         a.order = opt.order;
         a.limiter = opt.limiter;
         a.riemann = opt.riemann;
-        a.gas = luna::Gas{opt.gamma, opt.smallr, opt.smallc, 1.0 / (opt.gamma - 1.0)};
+        a.gas = luna::make_gas(opt.gamma, opt.smallr, opt.smallc);
         a.key = keys.p;
         a.period = period;
         a.step = step;
@@ -1581,6 +1582,20 @@ int order_line(luna_fv1* fv, unsigned long long descents, bool* sorted) {
     LUNA_HIP(luna::launch_line_sort(fv->stream, fv->line_key[fv->cur].p + fv->lo, fv->line_id.p + fv->lo, n, fv->packed.p, fv->sort_temp.p,
                                     &bytes));
     fv->sorts += 1;
+    return LUNA_OK;
+}
+
+// Waits for the time step that the fused kernel writes to host[0] (LINE_NO_STEP before the launch, a value no time step has):
+// watches the word for up to a millisecond, then waits for the stream, which also reports what went wrong with it.
+constexpr unsigned long long LINE_NO_STEP = ~0ull;
+int await_line_step(luna_fv1* fv) {
+    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
+    for (int k = 1;; ++k) {
+        if (__atomic_load_n(fv->host, __ATOMIC_ACQUIRE) != LINE_NO_STEP) return LUNA_OK;
+        if (k % 64 == 0 && std::chrono::steady_clock::now() > until) break;
+    }
+    LUNA_HIP(hipStreamSynchronize(fv->stream));
+    if (__atomic_load_n(fv->host, __ATOMIC_ACQUIRE) == LINE_NO_STEP) return fail(LUNA_ERR_DEVICE, "luna: the line's step left no time step");
     return LUNA_OK;
 }
 
@@ -1831,7 +1846,7 @@ int luna_fv1_time_step(luna_fv1* fv, double courant, int rule, double* dt) {
 int luna_fv1_step(luna_fv1* fv, double dt) {
     if (!fv) return fail(LUNA_ERR_ARGUMENT, "luna_fv1_step: null argument");
     if (!fv->moving) {
-        LUNA_HIP(luna::launch_line_step(fv->stream, fv->args(), dt, 0.0, false, fv->counters_now()));
+        LUNA_HIP(luna::launch_line_step(fv->stream, fv->args(), dt, 0.0, false, fv->counters_now(), fv->counters.p + 2, fv->host));
         std::swap(fv->q, fv->next);
         return LUNA_OK;
     }
@@ -1902,11 +1917,11 @@ int luna_fv1_step_and_time_step(luna_fv1* fv, double dt, double courant, double*
         if (again) return luna_fv1_time_step(fv, courant, LUNA_STEP_LUNA, next);
         return LUNA_OK;
     }
-    LUNA_HIP(luna::launch_line_step(fv->stream, fv->args(), dt, courant, true, fv->counters_now()));
+    fv->host[0] = LINE_NO_STEP;
+    LUNA_HIP(luna::launch_line_step(fv->stream, fv->args(), dt, courant, true, fv->counters_now(), fv->counters.p + 2, fv->host));
     fv->parity ^= 1;
     std::swap(fv->q, fv->next);
-    LUNA_HIP(hipMemcpyAsync(fv->host, fv->counters.p + slot, sizeof(unsigned long long), hipMemcpyDeviceToHost, fv->stream));
-    LUNA_HIP(hipStreamSynchronize(fv->stream));
+    if (int rc = await_line_step(fv)) return rc;
     *next = bits_to_double(fv->host[0]);
     return LUNA_OK;
 }

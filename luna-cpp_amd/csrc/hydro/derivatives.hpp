@@ -17,8 +17,7 @@ __device__ __forceinline__ int primitive_floors(const Gas& gas, const double* U)
     double v[D];
 #pragma unroll
     for (int k = 0; k < D; ++k) v[k] = U[1 + k] * inv_rho;
-    const double smalle = gas.smallc * gas.smallc / gas.gamma / (gas.gamma - 1.0);
-    return (U[0] >= gas.smallr ? 0 : 1) | (U[D + 1] - 0.5 * rho * dot<D>(v, v) >= smalle * rho ? 0 : 2);
+    return (U[0] >= gas.smallr ? 0 : 1) | (U[D + 1] - 0.5 * rho * dot<D>(v, v) >= gas.smalle * rho ? 0 : 2);
 }
 
 // euler.hpp:128-140: a floored density or energy has derivative zero in what the floor replaced.
@@ -32,9 +31,8 @@ __device__ __forceinline__ void primitive_tangent(const Gas& gas, const double* 
     for (int k = 0; k < D; ++k) v[k] = U[1 + k] * inv_rho;
 #pragma unroll
     for (int k = 0; k < D; ++k) dv[k] = (dU[1 + k] - v[k] * drho) * inv_rho;
-    const double smalle = gas.smallc * gas.smallc / gas.gamma / (gas.gamma - 1.0);
     const double dkinetic = 0.5 * drho * dot<D>(v, v) + rho * dot<D>(v, dv);
-    const double de = (floors & 2) ? smalle * drho : dU[D + 1] - dkinetic;
+    const double de = (floors & 2) ? gas.smalle * drho : dU[D + 1] - dkinetic;
     dW[0] = drho;
 #pragma unroll
     for (int k = 0; k < D; ++k) dW[1 + k] = dv[k];
@@ -52,11 +50,10 @@ __device__ __forceinline__ void primitive_adjoint(const Gas& gas, const double* 
         v[k] = U[1 + k] * inv_rho;
         vbar[k] = Wbar[1 + k];
     }
-    const double smalle = gas.smallc * gas.smallc / gas.gamma / (gas.gamma - 1.0);
     const double ebar = (gas.gamma - 1.0) * Wbar[D + 1];
     double rhobar = Wbar[0], energybar = 0.0;
     if (floors & 2) {
-        rhobar += smalle * ebar;  // e = smalle rho
+        rhobar += gas.smalle * ebar;  // e = smalle rho
     } else {                      // e = E - rho v.v / 2
         energybar = ebar;
         rhobar -= 0.5 * dot<D>(v, v) * ebar;

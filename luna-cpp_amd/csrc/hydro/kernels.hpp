@@ -254,7 +254,10 @@ struct LineArgs {
     long long* key_next;  // by slot: the key of the slot's point after the step
 };
 hipError_t launch_line_time_step(hipStream_t s, const LineArgs& a, double courant, int luna_rule, const Counters& c);
-hipError_t launch_line_step(hipStream_t s, const LineArgs& a, double dt, double courant, bool fused, const Counters& c);
+// The static step; fused, also the next dt by LUNA's rule into c.dt and, when the kernel is done, into *host (pinned host
+// memory). done: a word of device memory that is zero between launches.
+hipError_t launch_line_step(hipStream_t s, const LineArgs& a, double dt, double courant, bool fused, const Counters& c,
+                            unsigned long long* done, unsigned long long* host);
 // The moving step: Q, positions and keys after the step into a.next, a.x_next, a.key_next; the count of adjacent slots
 // out of order after the move into *descents (*descents_next reset for the next step); fused, the next dt by LUNA's rule.
 hipError_t launch_line_step_moving(hipStream_t s, const LineArgs& a, double dt, double courant, bool fused, const Counters& c,

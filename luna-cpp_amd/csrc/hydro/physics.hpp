@@ -12,7 +12,11 @@ namespace luna {
 
 struct Gas {
     double gamma, smallr, smallc, inverse_gm1;
+    double smalle;  // the floor of the specific internal energy, smallc^2 / gamma / (gamma - 1): two divisions, taken once on the host
 };
+inline Gas make_gas(double gamma, double smallr, double smallc) {
+    return Gas{gamma, smallr, smallc, 1.0 / (gamma - 1.0), smallc * smallc / gamma / (gamma - 1.0)};
+}
 
 // euler.hpp:69-73: left to right, written out per D.
 template <int D>
@@ -37,9 +41,8 @@ __device__ __forceinline__ void primitive(const Gas& gas, const double* U, doubl
     double v[D];
 #pragma unroll
     for (int k = 0; k < D; ++k) v[k] = U[1 + k] * inv_rho;
-    const double smalle = gas.smallc * gas.smallc / gas.gamma / (gas.gamma - 1.0);
     const double kinetic = 0.5 * rho * dot<D>(v, v);
-    const double e = fmax(U[D + 1] - kinetic, smalle * rho);
+    const double e = fmax(U[D + 1] - kinetic, gas.smalle * rho);
     W[0] = rho;
 #pragma unroll
     for (int k = 0; k < D; ++k) W[1 + k] = v[k];
