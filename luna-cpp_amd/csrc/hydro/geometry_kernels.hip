@@ -22,11 +22,20 @@ namespace {
 
 constexpr int BLOCK = 256;
 
+// The logical block of this work-group: work-groups go to the 8 XCDs in turn (block b to XCD b mod 8), so XCD x takes a
+// contiguous run, and the faces that neighbouring cells share are fetched into one L2.
+__device__ __forceinline__ int xcd_block() {
+    const int b = blockIdx.x, n = gridDim.x;
+    const int q = n >> 3, rem = n & 7, x = b & 7, k = b >> 3;
+    return x * q + min(x, rem) + k;
+}
+
 __device__ __forceinline__ void flag(unsigned int* flags, unsigned int bit) { atomicOr(flags, bit); }
 
 template <int D>
 __global__ __launch_bounds__(SLICE) void k_geo_cells(MeshIn m, double* cell, double* volume, int* count, int* longest, unsigned int* flags) {
     using C = CellAt<D>;
+    __shared__ double2 halves[SLICE][GEO_ROW / 2];
     const int i = blockIdx.x * SLICE + threadIdx.x;
     const long long E = 2LL * m.F;
     int n = 0;
@@ -50,9 +59,16 @@ __global__ __launch_bounds__(SLICE) void k_geo_cells(MeshIn m, double* cell, dou
         row[C::VOL] = v;
         volume[i] = v;
         row[C::RAD] = cell_radius<D>(v);
-        double* out = cell + (size_t)i * CELL_ROW;
 #pragma unroll
-        for (int k = 0; k < GEO_ROW; ++k) out[k] = row[k];
+        for (int k = 0; k < GEO_ROW; k += 2) halves[threadIdx.x][(k / 2) ^ (threadIdx.x & 3)] = make_double2(row[k], row[k + 1]);
+    }
+    __syncthreads();
+    // four lanes to a half row, so that a store covers whole runs of 64 B (lane by lane each 16 B touched a line of its own)
+#pragma unroll
+    for (int k = 0; k < GEO_ROW / 2; ++k) {
+        const int c = k * 16 + threadIdx.x / 4, q = threadIdx.x & 3;
+        if (blockIdx.x * SLICE + c < m.N)
+            reinterpret_cast<double2*>(cell + (size_t)(blockIdx.x * SLICE + c) * CELL_ROW)[q] = halves[c][q ^ (c & 3)];
     }
     // the slice's longest list (one wavefront per work-group)
 #pragma unroll
@@ -150,7 +166,11 @@ __global__ __launch_bounds__(BLOCK) void k_geo_pairs(MeshIn m, unsigned int* fla
 // writes each (entry t, array) as one whole run of 16 slots (one 128-byte line for the doubles). Padding slots (t at or
 // past the cell's list length) get zeros. A quarter deeper than QUARTER_DEPTH entries writes the rest straight to memory.
 // The CSR offsets were checked by k_geo_cells (the host runs this only when they passed).
-constexpr int SLOT_BLOCK = 256, QUARTER = 16, QUARTER_DEPTH = 48;
+// What bounds it is the latency of an entry's chain (list, cells, face arrays), so the wavefronts in flight: 32 entries deep
+// (20 KiB of LDS, 8 work-groups a CU) takes 0.46 ms at 104^3, 48 deep (5 a CU) 0.51; before, with the cells' own positions and
+// centroids read per entry, slices spread over the XCDs and stores that the L2 kept, 0.54. The stores bypass the L2
+// (nothing reads the slots before the sweep), which leaves it to the faces: the sweep after it 0.437 -> 0.425 ms.
+constexpr int SLOT_BLOCK = 256, QUARTER = 16, QUARTER_DEPTH = 32;
 template <int D>
 __global__ __launch_bounds__(SLOT_BLOCK) void k_geo_slots(MeshIn m, const int* __restrict__ count, const int* __restrict__ slice,
                                                           const long long* __restrict__ info, int S, int* __restrict__ list,
@@ -158,11 +178,16 @@ __global__ __launch_bounds__(SLOT_BLOCK) void k_geo_slots(MeshIn m, const int* _
     __shared__ int offs[QUARTER + 1];
     __shared__ int s_list[QUARTER_DEPTH * QUARTER], s_other[QUARTER_DEPTH * QUARTER];
     __shared__ double s_geo[D + 1][QUARTER_DEPTH * QUARTER];
-    const int g = blockIdx.x >> 2, quarter = blockIdx.x & 3;
+    __shared__ double s_pos[QUARTER * D], s_cen[QUARTER * D];  // the work-group's cells: every entry needs its cell's
+    const int block = xcd_block(), g = block >> 2, quarter = block & 3;
     const int c0 = g * SLICE + quarter * QUARTER, cells = max(0, min(QUARTER, m.N - c0));
     const int tid = threadIdx.x;
     if (cells > 0)
         for (int l = tid; l <= cells; l += SLOT_BLOCK) offs[l] = m.start[c0 + l];
+    for (int l = tid; l < cells * D; l += SLOT_BLOCK) {
+        s_pos[l] = m.positions[(size_t)c0 * D + l];
+        s_cen[l] = m.centroid[(size_t)c0 * D + l];
+    }
     const long long slots = info[0];
     const long long base = slice[g];
     const long long end = g + 1 < S ? (long long)slice[g + 1] : slots;
@@ -178,7 +203,6 @@ __global__ __launch_bounds__(SLOT_BLOCK) void k_geo_slots(MeshIn m, const int* _
     const int k0 = cells > 0 ? offs[0] : 0, k1 = cells > 0 ? offs[cells] : 0;
     const int* __restrict__ in_list = m.list;
     const double* __restrict__ pos = m.positions;
-    const double* __restrict__ cen = m.centroid;
     unsigned int bad = 0;
     for (int k = k0 + tid; k < k1; k += SLOT_BLOCK) {
         int lane = 0;  // the last l with offs[l] <= k
@@ -218,12 +242,12 @@ __global__ __launch_bounds__(SLOT_BLOCK) void k_geo_slots(MeshIn m, const int* _
                 if (e < 0) {
 #pragma unroll
                     for (int a = 0; a < D; ++a) {
-                        const double d = pos[(size_t)o * D + a] - pos[(size_t)i * D + a];
-                        rel[a] = rel[a] + (d - m.side[a] * round(d * m.inverse[a]));
+                        const double d = pos[(size_t)o * D + a] - s_pos[lane * D + a];
+                        rel[a] = rel[a] + wrap(d, m.side[a], m.inverse[a]);
                     }
                 }
 #pragma unroll
-                for (int a = 0; a < D; ++a) off[a] = rel[a] - cen[(size_t)i * D + a];
+                for (int a = 0; a < D; ++a) off[a] = rel[a] - s_cen[lane * D + a];
             }
         }
         if (t < QUARTER_DEPTH) {
@@ -247,11 +271,11 @@ __global__ __launch_bounds__(SLOT_BLOCK) void k_geo_slots(MeshIn m, const int* _
     for (int p = tid; p < staged * QUARTER; p += SLOT_BLOCK) {
         const int t = p / QUARTER, l = p % QUARTER;
         const long long sl = base + (long long)t * SLICE + quarter * QUARTER + l;
-        list[sl] = s_list[p];
-        other[sl] = s_other[p];
-        slot[sl] = s_geo[0][p];
+        __builtin_nontemporal_store(s_list[p], list + sl);
+        __builtin_nontemporal_store(s_other[p], other + sl);
+        __builtin_nontemporal_store(s_geo[0][p], slot + sl);
 #pragma unroll
-        for (int a = 0; a < D; ++a) slot[(a + 1) * slots + sl] = s_geo[1 + a][p];
+        for (int a = 0; a < D; ++a) __builtin_nontemporal_store(s_geo[1 + a][p], slot + (a + 1) * slots + sl);
     }
     for (int p = staged * QUARTER + tid; p < depth * QUARTER; p += SLOT_BLOCK) {
         const int t = p / QUARTER, l = p % QUARTER;
