@@ -7,6 +7,7 @@
 
 #include "derivatives.hpp"
 #include "kernels.hpp"
+#include "staged.hpp"
 
 namespace luna {
 namespace {
@@ -31,12 +32,6 @@ __device__ __forceinline__ int xcd_block() {
 }
 
 __device__ __forceinline__ int first_slot(const Geo& g, int i) { return g.slice[i >> 6] + (i & (SLICE - 1)); }
-
-template <int D>
-__device__ __forceinline__ void load_vec(const double* p, double* v) {
-#pragma unroll
-    for (int a = 0; a < D; ++a) v[a] = p[a];
-}
 
 template <int D>
 __device__ __forceinline__ void separation(const Geo& g, const double* xi, const double* xj, double* d) {
@@ -280,52 +275,47 @@ __device__ __forceinline__ void face_in(const Geo& g, int f, FaceIn<D>& x) {
     x.mag = sqrt(dot<D>(x.A, x.A));
 }
 
+// One side's state at the face: half step + g.r, the cell's own where its density or pressure would not stay positive
+// (returns whether).
+template <int D, class Side>
+__device__ __forceinline__ bool face_state(const Gas& gas, const Side& side, const double* off, double dt, double* out) {
+    constexpr int V = D + 2;
+    double W[V], gr[V * D];
+    side.state(W);
+    load_gradient<D>(side, gr);
+    half_step<D>(gas, W, gr, dt, out);
+#pragma unroll
+    for (int v = 0; v < V; ++v) out[v] += dot<D>(gr + v * D, off);
+    const bool fallback = !(out[0] > 0 && out[D + 1] > 0);
+    if (fallback)
+#pragma unroll
+        for (int v = 0; v < V; ++v) out[v] = W[v];
+    return fallback;
+}
+
 // One face's two sides as the static flux computes them (half step + g.r, positivity fallback), with their fallback
 // flags, offsets, the unit normal and |A|.
-template <int D>
-__device__ __forceinline__ void face_sides(const Geo& g, const Rows& r, const Gas& gas, const FaceIn<D>& face, double dt, double* Ls, double* Rs,
-                                           bool* fallback, double* ro, double* rj, double* n, double& magnitude) {
-    constexpr int V = D + 2;
-    using C = CellAt<D>;
-    const int2 pair = face.pair;
+template <int D, class SideO, class SideJ>
+__device__ __forceinline__ void face_sides(const Geo& g, const Gas& gas, const FaceIn<D>& face, const SideO& so, const SideJ& sj, double dt,
+                                           double* Ls, double* Rs, bool* fallback, double* ro, double* rj, double* n, double& magnitude) {
     magnitude = face.mag;
     const double inv = 1.0 / magnitude;
 #pragma unroll
     for (int k = 0; k < D; ++k) n[k] = face.A[k] * inv;
-    const double* ro_row = g.cell + (size_t)pair.x * CELL_ROW;
-    const double* rj_row = g.cell + (size_t)pair.y * CELL_ROW;
-    double xo[D], xj[D], d[D];
-    load_vec<D>(ro_row + C::X, xo);
-    load_vec<D>(rj_row + C::X, xj);
+    double xo[D], xj[D], co[D], cj[D], d[D];
+    so.place(xo, co);
+    sj.place(xj, cj);
     separation<D>(g, xj, xo, d);  // the owner seen from the neighbour
     const double half = 0.5 * dt, wf = 0.0;
 #pragma unroll
     for (int k = 0; k < D; ++k) {
-        ro[k] = face.fc[k] - ro_row[C::C + k];
-        rj[k] = face.fc[k] + d[k] - rj_row[C::C + k];
+        ro[k] = face.fc[k] - co[k];
+        rj[k] = face.fc[k] + d[k] - cj[k];
         ro[k] = ro[k] + wf * half;
         rj[k] = rj[k] + wf * half;
     }
-    const int cells[2] = {pair.x, pair.y};
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        double* out = s == 0 ? Ls : Rs;
-        const double* rs = s == 0 ? ro : rj;
-        const double* W = g.cell + (size_t)cells[s] * CELL_ROW + C::W;
-        const double* gr = r.grad + (size_t)cells[s] * grad_row<D>();
-        double Wc[V], gc[V * D];
-#pragma unroll
-        for (int v = 0; v < V; ++v) Wc[v] = W[v];
-#pragma unroll
-        for (int k = 0; k < V * D; ++k) gc[k] = gr[k];
-        half_step<D>(gas, Wc, gc, dt, out);
-#pragma unroll
-        for (int v = 0; v < V; ++v) out[v] += dot<D>(gc + v * D, rs);
-        fallback[s] = !(out[0] > 0 && out[D + 1] > 0);
-        if (fallback[s])
-#pragma unroll
-            for (int v = 0; v < V; ++v) out[v] = Wc[v];
-    }
+    fallback[0] = face_state<D>(gas, so, ro, dt, Ls);
+    fallback[1] = face_state<D>(gas, sj, rj, dt, Rs);
 }
 
 // ---- tangent ----
@@ -391,19 +381,60 @@ __global__ __launch_bounds__(BLOCK, LUNA_DERIV_WAVES) void k_fit_tangent(Geo g, 
     }
 }
 
-// One face's flux row and its tangent (x |A|).
+// One side's tangent: the half step's and g.r's, or the cell's own where its state is. dg: the gradient tangent's chunks.
+template <int D, class Side, class Chunks>
+__device__ __forceinline__ void side_tangent(const Gas& gas, const Side& side, const Chunks& dg, const double* dWi, bool fallback, const double* off,
+                                             double dt, double* out) {
+    constexpr int V = D + 2;
+    if (fallback) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) out[v] = dWi[v];
+        return;
+    }
+    double W[V], gi[V * D], dgi[V * D];
+    side.state(W);
+    load_gradient<D>(side, gi);
+#pragma unroll
+    for (int k = 0; k < V * D; k += 2) {
+        const double2v d = dg(k / 2);
+        dgi[k] = d.x;
+        if (k + 1 < V * D) dgi[k + 1] = d.y;
+    }
+    half_step_tangent<D>(gas, W, dWi, gi, dgi, dt, out);
+#pragma unroll
+    for (int v = 0; v < V; ++v) out[v] += dot<D>(dgi + v * D, off);
+}
+
+// One face's flux row and its tangent (x |A|), side by side (2V doubles a face), so that the update gathers one row per entry.
+// The neighbours' rows and gradient tangents come through LDS in whole lines (22 KiB a wavefront), the owners' are read in
+// place: @FLUXT@
 template <int D>
 __global__ __launch_bounds__(BLOCK) void k_flux_tangent(Geo g, Rows r, Gas gas, int riemann, double dt, const double* dW, const double* dgrad,
                                                         double* dflux) {
-    constexpr int V = D + 2, GR = grad_row<D>();
-    using C = CellAt<D>;
-    const int f = blockIdx.x * BLOCK + threadIdx.x;
+    constexpr int V = D + 2;
+    using Staged = StagedSide<D, 0>;
+    constexpr int GRAD = Staged::GRAD;
+    __shared__ double rows[Staged::DOUBLES + 64 * 2 * GRAD];
+    lds_double* lds = (lds_double*)rows;
+    lds_double* tangents = lds + Staged::DOUBLES;
+    const int lane = threadIdx.x, f = blockIdx.x * BLOCK + lane, at = min(f, g.F - 1);
+    const int j = g.neighbour[at];
+    Staged::fetch(g, r, j, true, lds, lane);
+    Staged::fetch_gradients(dgrad, j, tangents, lane);
+    FaceIn<D> face;
+    face_in<D>(g, at, face);
+    const MemorySide<D, 0> so(g, r, face.pair.x);
+    const Staged sj(lds, lane);
+    double dWo[V], dWj[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        dWo[v] = dW[(size_t)face.pair.x * V + v];
+        dWj[v] = dW[(size_t)j * V + v];
+    }
+    Staged::finish();
     if (f >= g.F) return;
-    // the face's flux and its tangent side by side (2V doubles a face), so that the update gathers one row per entry
     double* Fv = dflux + (size_t)f * 2 * V;
     double* dF = Fv + V;
-    FaceIn<D> face;
-    face_in<D>(g, f, face);
     if (face.mag == 0) {
 #pragma unroll
         for (int v = 0; v < V; ++v) Fv[v] = dF[v] = 0;
@@ -411,34 +442,10 @@ __global__ __launch_bounds__(BLOCK) void k_flux_tangent(Geo g, Rows r, Gas gas, 
     }
     double Ls[V], Rs[V], ro[D], rj[D], n[D], magnitude, dLs[V], dRs[V];
     bool fallback[2];
-    face_sides<D>(g, r, gas, face, dt, Ls, Rs, fallback, ro, rj, n, magnitude);
-    const int2 pair = face.pair;
-    const int cells[2] = {pair.x, pair.y};
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        double* out = s == 0 ? dLs : dRs;
-        const int i = cells[s];
-        if (fallback[s]) {
-#pragma unroll
-            for (int v = 0; v < V; ++v) out[v] = dW[(size_t)i * V + v];
-            continue;
-        }
-        double W[V], dWi[V], gi[V * D], dgi[V * D];
-#pragma unroll
-        for (int v = 0; v < V; ++v) {
-            W[v] = g.cell[(size_t)i * CELL_ROW + C::W + v];
-            dWi[v] = dW[(size_t)i * V + v];
-        }
-#pragma unroll
-        for (int k = 0; k < V * D; ++k) {
-            gi[k] = r.grad[(size_t)i * GR + k];
-            dgi[k] = dgrad[(size_t)i * GR + k];
-        }
-        half_step_tangent<D>(gas, W, dWi, gi, dgi, dt, out);
-        const double* rs = s == 0 ? ro : rj;
-#pragma unroll
-        for (int v = 0; v < V; ++v) out[v] += dot<D>(dgi + v * D, rs);
-    }
+    face_sides<D>(g, gas, face, so, sj, dt, Ls, Rs, fallback, ro, rj, n, magnitude);
+    const double2v* dgo = reinterpret_cast<const double2v*>(dgrad) + (size_t)face.pair.x * GRAD;
+    side_tangent<D>(gas, so, [&](int k) { return dgo[k]; }, dWo, fallback[0], ro, dt, dLs);
+    side_tangent<D>(gas, sj, [&](int k) { return Staged::gradient_chunk(tangents, lane, k); }, dWj, fallback[1], rj, dt, dRs);
     const double w0[D] = {};
     double Fl[V], dFl[V];
     riemann_tangent<D>(riemann, gas, Ls, Rs, dLs, dRs, n, w0, Fl, dFl);
@@ -505,23 +512,30 @@ __global__ __launch_bounds__(BLOCK) void k_update_tangent(Geo g, Rows r, double 
 // ---- adjoint ----
 
 // Per face: the bars of its two sides, (L bar, R bar) = J^T Fbar of the Riemann solve, Fbar = (dt qbar_j - dt qbar_o) |A|.
+// The neighbours' rows through LDS, as the flux: 114 us at 56^3 before, now 97.
 template <int D>
 __global__ __launch_bounds__(BLOCK) void k_face_adjoint(Geo g, Rows r, Gas gas, int riemann, double dt, const double* qbar, double* sidebar) {
     constexpr int V = D + 2;
-    const int f = blockIdx.x * BLOCK + threadIdx.x;
+    using Staged = StagedSide<D, 0>;
+    __shared__ double rows[Staged::DOUBLES];
+    lds_double* lds = (lds_double*)rows;
+    const int lane = threadIdx.x, f = blockIdx.x * BLOCK + lane, at = min(f, g.F - 1);
+    Staged::fetch(g, r, g.neighbour[at], true, lds, lane);
+    FaceIn<D> face;
+    face_in<D>(g, at, face);
+    const int2 pair = face.pair;
+    double Fbar[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) Fbar[v] = (dt * qbar[(size_t)pair.y * V + v] - dt * qbar[(size_t)pair.x * V + v]) * face.mag;
+    Staged::finish();
     if (f >= g.F) return;
     double Lbar[V], Rbar[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) Lbar[v] = Rbar[v] = 0;
-    FaceIn<D> face;
-    face_in<D>(g, f, face);
     if (face.mag != 0) {
-        double Ls[V], Rs[V], ro[D], rj[D], n[D], magnitude, Fbar[V];
+        double Ls[V], Rs[V], ro[D], rj[D], n[D], magnitude;
         bool fallback[2];
-        face_sides<D>(g, r, gas, face, dt, Ls, Rs, fallback, ro, rj, n, magnitude);
-        const int2 pair = face.pair;
-#pragma unroll
-        for (int v = 0; v < V; ++v) Fbar[v] = (dt * qbar[(size_t)pair.y * V + v] - dt * qbar[(size_t)pair.x * V + v]) * magnitude;
+        face_sides<D>(g, gas, face, MemorySide<D, 0>(g, r, pair.x), Staged(lds, lane), dt, Ls, Rs, fallback, ro, rj, n, magnitude);
         const double w0[D] = {};
         riemann_adjoint<D>(riemann, gas, Ls, Rs, n, w0, Fbar, Lbar, Rbar);
     }
