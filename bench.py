@@ -454,9 +454,8 @@ def main():
                      "frac": achieved / HBM_PEAK_GBS, "traffic": measured_traffic("moving " + name, n),
                      "algorithmic_bytes_per_cell": per_cell, "avg_ms": avg_ms, "launches": launches,
                      "valu_floor_ms": valu_floor_ms("k_sweep<3, true, true, 1, 0, 0>", n, N) if name == "sweep" else None,
-                     "note": "the FP64 sweep's arithmetic (7430-8396 VALU instructions a cell, 46 IEEE divisions in its solve) "
-                             "bounds it at its VALU floor before HBM: at the floor it would move its algorithmic bytes at "
-                             "about half of 8 TB/s"},
+                     "note": "valu_floor_ms: the time of the sweep's VALU instructions alone; what bounds it is the gather of "
+                             "its neighbours' rows and that arithmetic together"},
         "cpu_baseline": cpu,
         "learned_vs_plain": learned_cmp,
         "precision_policies": policies,

@@ -16,8 +16,8 @@ constexpr int BLOCK = 64;  // one wavefront per work-group: the per-cell walks d
 
 inline dim3 grid_of(long long n) { return dim3((unsigned)((n + BLOCK - 1) / BLOCK)); }
 
-// The heaviest per-cell kernels (the fit's tangent, the cell adjoint) need every register a lane can hold; at 2 waves per
-// SIMD they spill a few bytes and run faster than at 1 (the compiler's choice without a floor).
+// The heaviest per-cell kernels (the fit's tangent, the cell adjoint) take most of the registers a lane can hold; at 2
+// waves per SIMD they fit without a spill and run faster than at 1 (the compiler's choice without a floor).
 #ifndef LUNA_DERIV_WAVES
 #define LUNA_DERIV_WAVES 2
 #endif

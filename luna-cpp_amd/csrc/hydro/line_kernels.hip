@@ -1,7 +1,8 @@
-// The 1D step on a sorted line (finite_volume_1d.hpp), one work-item per slot: the five-cell stencil in registers, three
-// limited gradients, two face states, two Riemann fluxes and the new state in one kernel; fused, the next time step by
-// LUNA's rule from the new state as a block min-reduction. On a moving line the same kernel also gives each point its
-// velocity, new position and key; the slots' order is checked in it and restored by a device radix sort when points
+// The 1D step on a sorted line (finite_volume_1d.hpp) in one kernel; fused, the next time step by LUNA's rule from the new
+// state as a min-reduction. Static: one cell per lane (its limited gradient, face states and right face's flux), the
+// neighbours' values by shuffles. Moving: one work-item per slot with the five-cell stencil in registers, three limited
+// gradients, two face states and two Riemann fluxes; the kernel also gives each point its velocity, new position and key;
+// the slots' order is checked in it and restored by a device radix sort when points
 // crossed, and the walls' new cells are split from the end cells. FP64, -ffp-contract=off.
 #include <hip/hip_runtime.h>
 #include <hipcub/device/device_radix_sort.hpp>
