@@ -43,17 +43,27 @@ struct FaceOut {
 
 // The topology of one face of a cell's polyhedron (polygon) for the geometry's derivative: the neighbour behind it, the
 // sign that makes its area positive, and its vertices in cycle order, each as the other generators whose bisectors meet
-// there (3D: va and vb, two; 2D: va, one per end, the neighbour of the adjacent edge).
+// there (3D: va and vb, two; 2D: va, one per end, the neighbour of the adjacent edge): entries first .. first + count - 1
+// of the cell's va and vb.
 struct FaceTopo {
-    int j, sigma;
+    int j, sigma, first, count;
+};
+struct CellTopo {
+    std::vector<FaceTopo> faces;
     std::vector<int> va, vb;
+
+    void clear() {
+        faces.clear();
+        va.clear();
+        vb.clear();
+    }
 };
 
 struct CellOut {
     double volume = 0, centroid[3] = {0, 0, 0};
     std::vector<FaceOut> faces;
     bool want_topo = false;
-    std::vector<FaceTopo> topo;
+    CellTopo topo;
 };
 
 double wrap(double d, double side) { return d - side * std::round(d / side); }
@@ -315,7 +325,7 @@ bool finish3(Poly3& P, const std::vector<Candidate>& cands, CellOut& cell, std::
     cell.topo.clear();
     double volume = 0, moment[3] = {0, 0, 0};
     static thread_local std::vector<int> seen;
-    static thread_local std::vector<int> other_a, other_b;
+    std::vector<int>&other_a = cell.topo.va, &other_b = cell.topo.vb;
     seen.assign(P.np, 0);
     for (int s = 0; s < P.nt; ++s)
         for (int e = 0; e < 3; ++e) {
@@ -329,8 +339,7 @@ bool finish3(Poly3& P, const std::vector<Candidate>& cands, CellOut& cell, std::
             // Walk the face of plane k: from triangle (k, x, y) on to the triangle holding the edge k -> y.
             double poly[MAXT][3];
             int count = 0, cur = s;
-            other_a.clear();
-            other_b.clear();
+            const int first = static_cast<int>(other_a.size());
             do {
                 int r = 0;
                 while (P.t[cur][r] != k) ++r;
@@ -366,8 +375,12 @@ bool finish3(Poly3& P, const std::vector<Candidate>& cands, CellOut& cell, std::
                 area = -area;
                 for (double& x : c) x = -x;
             }
-            if (!(area > 0)) continue;  // a face of no extent: no face
-            if (cell.want_topo) cell.topo.push_back(FaceTopo{P.pj[k], sigma, other_a, other_b});
+            if (!(area > 0)) {  // a face of no extent: no face
+                other_a.resize(first);
+                other_b.resize(first);
+                continue;
+            }
+            if (cell.want_topo) cell.topo.faces.push_back(FaceTopo{P.pj[k], sigma, first, static_cast<int>(other_a.size()) - first});
             FaceOut f;
             f.j = P.pj[k];
             f.area = area;
@@ -402,7 +415,9 @@ bool finish2(Poly2& P, CellOut& cell, std::string& why) {
         const double tri = 0.5 * length * h;
         if (cell.want_topo) {
             const double cross = P.v[i][0] * P.v[u][1] - P.v[i][1] * P.v[u][0];
-            cell.topo.push_back(FaceTopo{P.pj[k], cross < 0 ? -1 : 1, {P.pj[P.label[(i + P.m - 1) % P.m]], P.pj[P.label[u]]}, {}});
+            cell.topo.faces.push_back(FaceTopo{P.pj[k], cross < 0 ? -1 : 1, static_cast<int>(cell.topo.va.size()), 2});
+            cell.topo.va.push_back(P.pj[P.label[(i + P.m - 1) % P.m]]);
+            cell.topo.va.push_back(P.pj[P.label[u]]);
         }
         FaceOut f;
         f.j = P.pj[k];
@@ -656,7 +671,8 @@ inline V3 cross(V3 a, V3 b) { return {a[1] * b[2] - a[2] * b[1], a[2] * b[0] - a
 inline double cross2(V3 a, V3 b) { return a[0] * b[1] - a[1] * b[0]; }
 
 // Solves M y = r for the D x D matrix of rows m[0..D-1] (Gaussian elimination with partial pivoting); transpose: M^T y = r.
-void solve(int D, const V3* m, const double* r, double* y, bool transpose) {
+template <int D>
+inline void solve(const V3* m, const double* r, double* y, bool transpose) {
     double a[3][4];
     for (int p = 0; p < D; ++p) {
         for (int q = 0; q < D; ++q) a[p][q] = transpose ? m[q][p] : m[p][q];
@@ -680,53 +696,73 @@ void solve(int D, const V3* m, const double* r, double* y, bool transpose) {
     }
 }
 
+// The bars one cell's faces give its own position (entry 0) and those of the generators around it: some 17 sums, where the
+// single terms, one for each generator of each vertex of each face, would be 480 (15 KiB a cell written and read back).
+struct CellBars {
+    std::vector<std::pair<int, V3>> at;
+
+    void start(int i) { at.assign(1, {i, V3{0, 0, 0}}); }
+    // A term g of x_j - x_i.
+    void pull(int j, V3 g) {
+        size_t k = 1;
+        while (k < at.size() && at[k].first != j) ++k;
+        if (k == at.size()) at.push_back({j, V3{0, 0, 0}});
+        at[k].second = add(at[k].second, g);
+        at[0].second = sub(at[0].second, g);
+    }
+};
+
 }  // namespace
 
 struct luna_mesh_derivative {
     int D = 3, N = 0;
     double side[3] = {0, 0, 0};
     std::vector<double> x;                 // snapped positions
-    std::vector<std::vector<FaceTopo>> topo;
+    std::vector<CellTopo> topo;
     std::vector<std::vector<int>> face_id;  // per cell and topo face: the mesh's face row it gives (owner's kept faces), or -1
 
+    template <int D>
     V3 sep(int i, int j) const {
         V3 d{0, 0, 0};
         for (int a = 0; a < D; ++a) d[a] = wrap(x[static_cast<size_t>(j) * D + a] - x[static_cast<size_t>(i) * D + a], side[a]);
         return d;
     }
+    template <int D>
     V3 row(const double* p, int i) const {
         V3 r{0, 0, 0};
         for (int a = 0; a < D; ++a) r[a] = p[static_cast<size_t>(i) * D + a];
         return r;
     }
     // The vertex of cell i on the bisectors of js[0..D-1] (relative to x_i), with the rows it solved.
+    template <int D>
     V3 vertex(int i, const int* js, V3* m) const {
         double r[3];
         for (int p = 0; p < D; ++p) {
-            m[p] = sep(i, js[p]);
+            m[p] = sep<D>(i, js[p]);
             r[p] = 0.5 * dot3(m[p], m[p]);
         }
         double y[3] = {0, 0, 0};
-        solve(D, m, r, y, false);
+        solve<D>(m, r, y, false);
         return {y[0], y[1], D == 3 ? y[2] : 0.0};
     }
     // dv from dx (tangent).
+    template <int D>
     V3 vertex_tangent(int i, const int* js, const V3* m, V3 v, const double* dx) const {
         double s[3];
-        for (int p = 0; p < D; ++p) s[p] = dot3(sub(row(dx, js[p]), row(dx, i)), sub(m[p], v));
+        for (int p = 0; p < D; ++p) s[p] = dot3(sub(row<D>(dx, js[p]), row<D>(dx, i)), sub(m[p], v));
         double y[3] = {0, 0, 0};
-        solve(D, m, s, y, false);
+        solve<D>(m, s, y, false);
         return {y[0], y[1], D == 3 ? y[2] : 0.0};
     }
-    // vbar -> the bars of x_i and the js (adjoint), into acc.
-    void vertex_adjoint(int i, const int* js, const V3* m, V3 v, V3 vbar, std::vector<std::pair<int, V3>>& acc) const {
+    // vbar -> the bars of x_i and the js (adjoint), added to the cell's.
+    template <int D>
+    void vertex_adjoint(const int* js, const V3* m, V3 v, V3 vbar, CellBars& bars) const {
         const double r[3] = {vbar[0], vbar[1], vbar[2]};
         double sbar[3] = {0, 0, 0};
-        solve(D, m, r, sbar, true);
+        solve<D>(m, r, sbar, true);
         for (int p = 0; p < D; ++p) {
             const V3 g = mul(sub(m[p], v), sbar[p]);
-            acc.push_back({js[p], g});
-            acc.push_back({i, mul(g, -1.0)});
+            bars.pull(js[p], g);
         }
     }
 };
@@ -749,11 +785,13 @@ extern "C" int luna_mesh_derivative_create(const luna_mesh_record* mesh, luna_me
     }
     g->topo.resize(g->N);
     g->face_id.resize(g->N);
+#pragma omp parallel for schedule(static)
     for (int i = 0; i < g->N; ++i) {
         g->topo[i] = std::move(cells[i].topo);
-        g->face_id[i].assign(g->topo[i].size(), -1);
-        for (size_t t = 0; t < g->topo[i].size(); ++t) {
-            const int j = g->topo[i][t].j;
+        const auto& faces = g->topo[i].faces;
+        g->face_id[i].assign(faces.size(), -1);
+        for (size_t t = 0; t < faces.size(); ++t) {
+            const int j = faces[t].j;
             if (j <= i) continue;
             for (int k = mesh->start[i]; k < mesh->start[i + 1]; ++k) {
                 const int e = mesh->list[k];
@@ -767,81 +805,238 @@ extern "C" int luna_mesh_derivative_create(const luna_mesh_record* mesh, luna_me
 
 extern "C" void luna_mesh_derivative_destroy(luna_mesh_derivative* g) { delete g; }
 
+namespace {
+
+template <int D>
+void geometry_tangent(const luna_mesh_derivative* g, const double* dx, double* dV, double* dc, double* dA, double* dxf) {
+#pragma omp parallel
+    {
+        std::vector<V3> w, dw;
+#pragma omp for schedule(dynamic, 64)
+        for (int i = 0; i < g->N; ++i) {
+            double V = 0, dVi = 0;
+            V3 moment{0, 0, 0}, dmoment{0, 0, 0};
+            const CellTopo& topo = g->topo[i];
+            const auto& faces = topo.faces;
+            for (size_t t = 0; t < faces.size(); ++t) {
+                const FaceTopo& F = faces[t];
+                const V3 d = g->sep<D>(i, F.j), dd = sub(g->row<D>(dx, F.j), g->row<D>(dx, i));
+                const double dist = std::sqrt(dot3(d, d)), ddist = dot3(d, dd) / dist;
+                const V3 n = mul(d, 1.0 / dist), dn = mul(sub(dd, mul(n, dot3(n, dd))), 1.0 / dist);
+                const int m = F.count;
+                const int *va = topo.va.data() + F.first, *vb = topo.vb.data() + (D == 3 ? F.first : 0);
+                w.resize(m);
+                dw.resize(m);
+                for (int q = 0; q < m; ++q) {
+                    const int js[3] = {F.j, va[q], D == 3 ? vb[q] : 0};
+                    V3 rows[3];
+                    w[q] = g->vertex<D>(i, js, rows);
+                    dw[q] = g->vertex_tangent<D>(i, js, rows, w[q], dx);
+                }
+                double area = 0, darea = 0, pyr, dpyr;
+                V3 fc, dfc;
+                if (D == 3) {
+                    V3 cnum{0, 0, 0}, dcnum{0, 0, 0};
+                    for (int q = 1; q + 1 < m; ++q) {
+                        const V3 a = sub(w[q], w[0]), b = sub(w[q + 1], w[0]), da = sub(dw[q], dw[0]), db = sub(dw[q + 1], dw[0]);
+                        const V3 cr = cross(a, b), dcr = add(cross(da, b), cross(a, db));
+                        const double tri = 0.5 * dot3(cr, n), dtri = 0.5 * (dot3(dcr, n) + dot3(cr, dn));
+                        const V3 gq = mul(add(add(w[0], w[q]), w[q + 1]), 1.0 / 3.0), dgq = mul(add(add(dw[0], dw[q]), dw[q + 1]), 1.0 / 3.0);
+                        area += tri;
+                        darea += dtri;
+                        cnum = add(cnum, mul(gq, tri));
+                        dcnum = add(dcnum, add(mul(gq, dtri), mul(dgq, tri)));
+                    }
+                    area *= F.sigma;
+                    darea *= F.sigma;
+                    cnum = mul(cnum, F.sigma);
+                    dcnum = mul(dcnum, F.sigma);
+                    fc = mul(cnum, 1.0 / area);
+                    dfc = mul(sub(dcnum, mul(fc, darea)), 1.0 / area);
+                    pyr = area * dist / 6.0;
+                    dpyr = (darea * dist + area * ddist) / 6.0;
+                    moment = add(moment, mul(fc, 0.75 * pyr));
+                    dmoment = add(dmoment, mul(add(mul(dfc, pyr), mul(fc, dpyr)), 0.75));
+                } else {
+                    const V3 e = sub(w[1], w[0]), de = sub(dw[1], dw[0]);
+                    area = std::sqrt(dot3(e, e));
+                    darea = dot3(e, de) / area;
+                    fc = mul(add(w[0], w[1]), 0.5);
+                    dfc = mul(add(dw[0], dw[1]), 0.5);
+                    pyr = 0.5 * F.sigma * cross2(w[0], w[1]);
+                    dpyr = 0.5 * F.sigma * (cross2(dw[0], w[1]) + cross2(w[0], dw[1]));
+                    moment = add(moment, mul(fc, (2.0 / 3.0) * pyr));
+                    dmoment = add(dmoment, mul(add(mul(dfc, pyr), mul(fc, dpyr)), 2.0 / 3.0));
+                }
+                V += pyr;
+                dVi += dpyr;
+                const int f = g->face_id[i][t];
+                if (f >= 0) {
+                    const V3 dAv = add(mul(n, darea), mul(dn, area));
+                    for (int a = 0; a < D; ++a) {
+                        dA[static_cast<size_t>(f) * D + a] = dAv[a];
+                        dxf[static_cast<size_t>(f) * D + a] = dfc[a];
+                    }
+                }
+            }
+            dV[i] = dVi;
+            const V3 c = mul(moment, 1.0 / V);
+            const V3 dci = mul(sub(dmoment, mul(c, dVi)), 1.0 / V);
+            for (int a = 0; a < D; ++a) dc[static_cast<size_t>(i) * D + a] = dci[a];
+        }
+    }
+}
+
+// What bounds it is the vertices' solves; each cell's bars are summed within the cell first (CellBars) and added in cell
+// order, the same sums every run. At 8000 cells and 8 threads, before: every single term kept for that pass (124 MB) and
+// vectors of each face's vertices allocated per face, 66 ms; now 20. The tangent, by the latter alone, 22 -> 13 ms; releasing
+// the topology, its rings two arrays of a cell instead of two of each face, 8.3 -> 2.6 ms.
+template <int D>
+void geometry_adjoint(const luna_mesh_derivative* g, const double* Vbar, const double* cbar, const double* Abar, const double* xfbar, double* xbar) {
+    const int N = g->N;
+    struct Face {
+        V3 d, n, fc;
+        double dist, area, pyr;
+    };
+    std::vector<std::vector<std::pair<int, V3>>> acc(N);
+#pragma omp parallel
+    {
+        std::vector<Face> fs;
+        std::vector<V3> ws, all_rows, wbar;  // per vertex of the cell's faces: it, the rows it solved; of one face: its bar
+        CellBars bars;
+#pragma omp for schedule(dynamic, 64)
+        for (int i = 0; i < N; ++i) {
+            const CellTopo& topo = g->topo[i];
+            const auto& faces = topo.faces;
+            bars.start(i);
+            // Forward: V, moment (the cell's own faces), then c = moment / V.
+            double V = 0;
+            V3 moment{0, 0, 0};
+            fs.resize(faces.size());
+            ws.resize(topo.va.size());
+            all_rows.resize(topo.va.size() * 3);
+            for (size_t t = 0; t < faces.size(); ++t) {
+                const FaceTopo& F = faces[t];
+                Face& s = fs[t];
+                s.d = g->sep<D>(i, F.j);
+                s.dist = std::sqrt(dot3(s.d, s.d));
+                s.n = mul(s.d, 1.0 / s.dist);
+                const int m = F.count;
+                const int *va = topo.va.data() + F.first, *vb = topo.vb.data() + (D == 3 ? F.first : 0);
+                V3 *w = ws.data() + F.first, *rows = all_rows.data() + static_cast<size_t>(F.first) * 3;
+                for (int q = 0; q < m; ++q) {
+                    const int js[3] = {F.j, va[q], D == 3 ? vb[q] : 0};
+                    w[q] = g->vertex<D>(i, js, rows + static_cast<size_t>(q) * 3);
+                }
+                if (D == 3) {
+                    double area = 0;
+                    V3 cnum{0, 0, 0};
+                    for (int q = 1; q + 1 < m; ++q) {
+                        const double tri = 0.5 * dot3(cross(sub(w[q], w[0]), sub(w[q + 1], w[0])), s.n);
+                        area += tri;
+                        cnum = add(cnum, mul(add(add(w[0], w[q]), w[q + 1]), tri / 3.0));
+                    }
+                    s.area = area * F.sigma;
+                    s.fc = mul(cnum, F.sigma / s.area);
+                    s.pyr = s.area * s.dist / 6.0;
+                    moment = add(moment, mul(s.fc, 0.75 * s.pyr));
+                } else {
+                    const V3 e = sub(w[1], w[0]);
+                    s.area = std::sqrt(dot3(e, e));
+                    s.fc = mul(add(w[0], w[1]), 0.5);
+                    s.pyr = 0.5 * F.sigma * cross2(w[0], w[1]);
+                    moment = add(moment, mul(s.fc, (2.0 / 3.0) * s.pyr));
+                }
+                V += s.pyr;
+            }
+            const V3 c = mul(moment, 1.0 / V);
+            // Reverse: c = moment / V.
+            const V3 cb = g->row<D>(cbar, i);
+            const V3 momentbar = mul(cb, 1.0 / V);
+            const double Vb = Vbar[i] - dot3(cb, c) / V;
+            const double share = D == 3 ? 0.75 : 2.0 / 3.0;
+            for (size_t t = 0; t < faces.size(); ++t) {
+                const FaceTopo& F = faces[t];
+                const Face& s = fs[t];
+                const int m = F.count;
+                const int *va = topo.va.data() + F.first, *vb = topo.vb.data() + (D == 3 ? F.first : 0);
+                const V3 *w = ws.data() + F.first, *rows = all_rows.data() + static_cast<size_t>(F.first) * 3;
+                double pyrbar = Vb + share * dot3(momentbar, s.fc);
+                V3 fcbar = mul(momentbar, share * s.pyr);
+                double areabar = 0, distbar = 0;
+                V3 nbar{0, 0, 0};
+                const int f = g->face_id[i][t];
+                if (f >= 0) {
+                    const V3 Ab = g->row<D>(Abar, f);
+                    areabar += dot3(Ab, s.n);
+                    nbar = add(nbar, mul(Ab, s.area));
+                    fcbar = add(fcbar, g->row<D>(xfbar, f));
+                }
+                wbar.assign(m, V3{0, 0, 0});
+                if (D == 3) {
+                    areabar += pyrbar * s.dist / 6.0;
+                    distbar += pyrbar * s.area / 6.0;
+                    // fc = cnum / area
+                    const V3 cnumbar = mul(fcbar, 1.0 / s.area);
+                    areabar -= dot3(fcbar, s.fc) / s.area;
+                    for (int q = 1; q + 1 < m; ++q) {
+                        const V3 a = sub(w[q], w[0]), b = sub(w[q + 1], w[0]);
+                        const V3 cr = cross(a, b);
+                        const double tri = 0.5 * dot3(cr, s.n);
+                        const V3 gq = mul(add(add(w[0], w[q]), w[q + 1]), 1.0 / 3.0);
+                        // area = sigma sum tri, cnum = sigma sum tri gq
+                        const double tribar = F.sigma * (areabar + dot3(cnumbar, gq));
+                        const V3 gbar = mul(cnumbar, F.sigma * tri / 3.0);
+                        wbar[0] = add(wbar[0], gbar);
+                        wbar[q] = add(wbar[q], gbar);
+                        wbar[q + 1] = add(wbar[q + 1], gbar);
+                        // tri = cr . n / 2
+                        const V3 crbar = mul(s.n, 0.5 * tribar);
+                        nbar = add(nbar, mul(cr, 0.5 * tribar));
+                        const V3 abar = cross(b, crbar), bbar = cross(crbar, a);
+                        wbar[q] = add(wbar[q], abar);
+                        wbar[q + 1] = add(wbar[q + 1], bbar);
+                        wbar[0] = sub(wbar[0], add(abar, bbar));
+                    }
+                } else {
+                    // pyr = sigma w0 x w1 / 2, fc = (w0 + w1) / 2, area = |w1 - w0|
+                    const double pb = 0.5 * F.sigma * pyrbar;
+                    wbar[0] = add(wbar[0], V3{pb * w[1][1], -pb * w[1][0], 0});
+                    wbar[1] = add(wbar[1], V3{-pb * w[0][1], pb * w[0][0], 0});
+                    wbar[0] = add(wbar[0], mul(fcbar, 0.5));
+                    wbar[1] = add(wbar[1], mul(fcbar, 0.5));
+                    const V3 e = sub(w[1], w[0]);
+                    const V3 eb = mul(e, areabar / s.area);
+                    wbar[1] = add(wbar[1], eb);
+                    wbar[0] = sub(wbar[0], eb);
+                }
+                // n = d / |d|, |d|
+                V3 dbar = add(mul(sub(nbar, mul(s.n, dot3(s.n, nbar))), 1.0 / s.dist), mul(s.n, distbar));
+                bars.pull(F.j, dbar);
+                for (int q = 0; q < m; ++q) {
+                    const int js[3] = {F.j, va[q], D == 3 ? vb[q] : 0};
+                    g->vertex_adjoint<D>(js, rows + static_cast<size_t>(q) * 3, w[q], wbar[q], bars);
+                }
+            }
+            acc[i] = bars.at;
+        }
+    }
+    for (int i = 0; i < N; ++i)  // in cell order: the same sums every run
+        for (const auto& p : acc[i])
+            for (int a = 0; a < D; ++a) xbar[static_cast<size_t>(p.first) * D + a] += p.second[a];
+}
+
+}  // namespace
+
 extern "C" int luna_mesh_derivative_tangent(const luna_mesh_derivative* g, const double* dx, double* dV, double* dc, double* dA, double* dxf) {
     if (!g || !dx || !dV || !dc || !dA || !dxf) {
         g_error = "luna_mesh_derivative_tangent: null argument";
         return 1;
     }
-    const int D = g->D;
-#pragma omp parallel for schedule(dynamic, 256)
-    for (int i = 0; i < g->N; ++i) {
-        double V = 0, dVi = 0;
-        V3 moment{0, 0, 0}, dmoment{0, 0, 0};
-        const auto& faces = g->topo[i];
-        for (size_t t = 0; t < faces.size(); ++t) {
-            const FaceTopo& F = faces[t];
-            const V3 d = g->sep(i, F.j), dd = sub(g->row(dx, F.j), g->row(dx, i));
-            const double dist = std::sqrt(dot3(d, d)), ddist = dot3(d, dd) / dist;
-            const V3 n = mul(d, 1.0 / dist), dn = mul(sub(dd, mul(n, dot3(n, dd))), 1.0 / dist);
-            const int m = static_cast<int>(F.va.size());
-            std::vector<V3> w(m), dw(m);
-            for (int q = 0; q < m; ++q) {
-                const int js[3] = {F.j, F.va[q], D == 3 ? F.vb[q] : 0};
-                V3 rows[3];
-                w[q] = g->vertex(i, js, rows);
-                dw[q] = g->vertex_tangent(i, js, rows, w[q], dx);
-            }
-            double area = 0, darea = 0, pyr, dpyr;
-            V3 fc, dfc;
-            if (D == 3) {
-                V3 cnum{0, 0, 0}, dcnum{0, 0, 0};
-                for (int q = 1; q + 1 < m; ++q) {
-                    const V3 a = sub(w[q], w[0]), b = sub(w[q + 1], w[0]), da = sub(dw[q], dw[0]), db = sub(dw[q + 1], dw[0]);
-                    const V3 cr = cross(a, b), dcr = add(cross(da, b), cross(a, db));
-                    const double tri = 0.5 * dot3(cr, n), dtri = 0.5 * (dot3(dcr, n) + dot3(cr, dn));
-                    const V3 gq = mul(add(add(w[0], w[q]), w[q + 1]), 1.0 / 3.0), dgq = mul(add(add(dw[0], dw[q]), dw[q + 1]), 1.0 / 3.0);
-                    area += tri;
-                    darea += dtri;
-                    cnum = add(cnum, mul(gq, tri));
-                    dcnum = add(dcnum, add(mul(gq, dtri), mul(dgq, tri)));
-                }
-                area *= F.sigma;
-                darea *= F.sigma;
-                cnum = mul(cnum, F.sigma);
-                dcnum = mul(dcnum, F.sigma);
-                fc = mul(cnum, 1.0 / area);
-                dfc = mul(sub(dcnum, mul(fc, darea)), 1.0 / area);
-                pyr = area * dist / 6.0;
-                dpyr = (darea * dist + area * ddist) / 6.0;
-                moment = add(moment, mul(fc, 0.75 * pyr));
-                dmoment = add(dmoment, mul(add(mul(dfc, pyr), mul(fc, dpyr)), 0.75));
-            } else {
-                const V3 e = sub(w[1], w[0]), de = sub(dw[1], dw[0]);
-                area = std::sqrt(dot3(e, e));
-                darea = dot3(e, de) / area;
-                fc = mul(add(w[0], w[1]), 0.5);
-                dfc = mul(add(dw[0], dw[1]), 0.5);
-                pyr = 0.5 * F.sigma * cross2(w[0], w[1]);
-                dpyr = 0.5 * F.sigma * (cross2(dw[0], w[1]) + cross2(w[0], dw[1]));
-                moment = add(moment, mul(fc, (2.0 / 3.0) * pyr));
-                dmoment = add(dmoment, mul(add(mul(dfc, pyr), mul(fc, dpyr)), 2.0 / 3.0));
-            }
-            V += pyr;
-            dVi += dpyr;
-            const int f = g->face_id[i][t];
-            if (f >= 0) {
-                const V3 dAv = add(mul(n, darea), mul(dn, area));
-                for (int a = 0; a < D; ++a) {
-                    dA[static_cast<size_t>(f) * D + a] = dAv[a];
-                    dxf[static_cast<size_t>(f) * D + a] = dfc[a];
-                }
-            }
-        }
-        dV[i] = dVi;
-        const V3 c = mul(moment, 1.0 / V);
-        const V3 dci = mul(sub(dmoment, mul(c, dVi)), 1.0 / V);
-        for (int a = 0; a < D; ++a) dc[static_cast<size_t>(i) * D + a] = dci[a];
-    }
+    if (g->D == 3)
+        geometry_tangent<3>(g, dx, dV, dc, dA, dxf);
+    else
+        geometry_tangent<2>(g, dx, dV, dc, dA, dxf);
     return 0;
 }
 
@@ -851,126 +1046,9 @@ extern "C" int luna_mesh_derivative_adjoint(const luna_mesh_derivative* g, const
         g_error = "luna_mesh_derivative_adjoint: null argument";
         return 1;
     }
-    const int D = g->D, N = g->N;
-    std::vector<std::vector<std::pair<int, V3>>> acc(N);
-#pragma omp parallel for schedule(dynamic, 256)
-    for (int i = 0; i < N; ++i) {
-        auto& out = acc[i];
-        const auto& faces = g->topo[i];
-        // Forward: V, moment (the cell's own faces), then c = moment / V.
-        double V = 0;
-        V3 moment{0, 0, 0};
-        struct Face {
-            V3 d, n, fc;
-            double dist, area, pyr;
-            std::vector<V3> w, rows;
-        };
-        std::vector<Face> fs(faces.size());
-        for (size_t t = 0; t < faces.size(); ++t) {
-            const FaceTopo& F = faces[t];
-            Face& s = fs[t];
-            s.d = g->sep(i, F.j);
-            s.dist = std::sqrt(dot3(s.d, s.d));
-            s.n = mul(s.d, 1.0 / s.dist);
-            const int m = static_cast<int>(F.va.size());
-            s.w.resize(m);
-            s.rows.resize(static_cast<size_t>(m) * 3);
-            for (int q = 0; q < m; ++q) {
-                const int js[3] = {F.j, F.va[q], D == 3 ? F.vb[q] : 0};
-                s.w[q] = g->vertex(i, js, &s.rows[static_cast<size_t>(q) * 3]);
-            }
-            if (D == 3) {
-                double area = 0;
-                V3 cnum{0, 0, 0};
-                for (int q = 1; q + 1 < m; ++q) {
-                    const double tri = 0.5 * dot3(cross(sub(s.w[q], s.w[0]), sub(s.w[q + 1], s.w[0])), s.n);
-                    area += tri;
-                    cnum = add(cnum, mul(add(add(s.w[0], s.w[q]), s.w[q + 1]), tri / 3.0));
-                }
-                s.area = area * F.sigma;
-                s.fc = mul(cnum, F.sigma / s.area);
-                s.pyr = s.area * s.dist / 6.0;
-                moment = add(moment, mul(s.fc, 0.75 * s.pyr));
-            } else {
-                const V3 e = sub(s.w[1], s.w[0]);
-                s.area = std::sqrt(dot3(e, e));
-                s.fc = mul(add(s.w[0], s.w[1]), 0.5);
-                s.pyr = 0.5 * F.sigma * cross2(s.w[0], s.w[1]);
-                moment = add(moment, mul(s.fc, (2.0 / 3.0) * s.pyr));
-            }
-            V += s.pyr;
-        }
-        const V3 c = mul(moment, 1.0 / V);
-        // Reverse: c = moment / V.
-        const V3 cb = g->row(cbar, i);
-        const V3 momentbar = mul(cb, 1.0 / V);
-        const double Vb = Vbar[i] - dot3(cb, c) / V;
-        const double share = D == 3 ? 0.75 : 2.0 / 3.0;
-        for (size_t t = 0; t < faces.size(); ++t) {
-            const FaceTopo& F = faces[t];
-            const Face& s = fs[t];
-            const int m = static_cast<int>(s.w.size());
-            double pyrbar = Vb + share * dot3(momentbar, s.fc);
-            V3 fcbar = mul(momentbar, share * s.pyr);
-            double areabar = 0, distbar = 0;
-            V3 nbar{0, 0, 0};
-            const int f = g->face_id[i][t];
-            if (f >= 0) {
-                const V3 Ab = g->row(Abar, f);
-                areabar += dot3(Ab, s.n);
-                nbar = add(nbar, mul(Ab, s.area));
-                fcbar = add(fcbar, g->row(xfbar, f));
-            }
-            std::vector<V3> wbar(m, V3{0, 0, 0});
-            if (D == 3) {
-                areabar += pyrbar * s.dist / 6.0;
-                distbar += pyrbar * s.area / 6.0;
-                // fc = cnum / area
-                const V3 cnumbar = mul(fcbar, 1.0 / s.area);
-                areabar -= dot3(fcbar, s.fc) / s.area;
-                for (int q = 1; q + 1 < m; ++q) {
-                    const V3 a = sub(s.w[q], s.w[0]), b = sub(s.w[q + 1], s.w[0]);
-                    const V3 cr = cross(a, b);
-                    const double tri = 0.5 * dot3(cr, s.n);
-                    const V3 gq = mul(add(add(s.w[0], s.w[q]), s.w[q + 1]), 1.0 / 3.0);
-                    // area = sigma sum tri, cnum = sigma sum tri gq
-                    const double tribar = F.sigma * (areabar + dot3(cnumbar, gq));
-                    const V3 gbar = mul(cnumbar, F.sigma * tri / 3.0);
-                    wbar[0] = add(wbar[0], gbar);
-                    wbar[q] = add(wbar[q], gbar);
-                    wbar[q + 1] = add(wbar[q + 1], gbar);
-                    // tri = cr . n / 2
-                    const V3 crbar = mul(s.n, 0.5 * tribar);
-                    nbar = add(nbar, mul(cr, 0.5 * tribar));
-                    const V3 abar = cross(b, crbar), bbar = cross(crbar, a);
-                    wbar[q] = add(wbar[q], abar);
-                    wbar[q + 1] = add(wbar[q + 1], bbar);
-                    wbar[0] = sub(wbar[0], add(abar, bbar));
-                }
-            } else {
-                // pyr = sigma w0 x w1 / 2, fc = (w0 + w1) / 2, area = |w1 - w0|
-                const double pb = 0.5 * F.sigma * pyrbar;
-                wbar[0] = add(wbar[0], V3{pb * s.w[1][1], -pb * s.w[1][0], 0});
-                wbar[1] = add(wbar[1], V3{-pb * s.w[0][1], pb * s.w[0][0], 0});
-                wbar[0] = add(wbar[0], mul(fcbar, 0.5));
-                wbar[1] = add(wbar[1], mul(fcbar, 0.5));
-                const V3 e = sub(s.w[1], s.w[0]);
-                const V3 eb = mul(e, areabar / s.area);
-                wbar[1] = add(wbar[1], eb);
-                wbar[0] = sub(wbar[0], eb);
-            }
-            // n = d / |d|, |d|
-            V3 dbar = add(mul(sub(nbar, mul(s.n, dot3(s.n, nbar))), 1.0 / s.dist), mul(s.n, distbar));
-            out.push_back({F.j, dbar});
-            out.push_back({i, mul(dbar, -1.0)});
-            for (int q = 0; q < m; ++q) {
-                const int js[3] = {F.j, F.va[q], D == 3 ? F.vb[q] : 0};
-                g->vertex_adjoint(i, js, &s.rows[static_cast<size_t>(q) * 3], s.w[q], wbar[q], out);
-            }
-        }
-    }
-    for (int i = 0; i < N; ++i)  // in cell order: the same sums every run
-        for (const auto& p : acc[i])
-            for (int a = 0; a < D; ++a) xbar[static_cast<size_t>(p.first) * D + a] += p.second[a];
+    if (g->D == 3)
+        geometry_adjoint<3>(g, Vbar, cbar, Abar, xfbar, xbar);
+    else
+        geometry_adjoint<2>(g, Vbar, cbar, Abar, xfbar, xbar);
     return 0;
 }

@@ -140,3 +140,34 @@ def test_geometry_derivative_against_the_producer(D, n):
     lhs = sum(np.sum(b * t) for b, t in zip(bars, (dV, dc, dA, dxf)))
     assert abs(lhs - np.sum(xbar * dx)) < 1e-12 * abs(lhs)
     g.close()
+
+
+@pytest.mark.parametrize("D,n,jitter", [(2, 8, 0.0), (2, 11, 0.45), (2, 23, 0.25), (3, 5, 0.4), (3, 6, 0.1), (3, 9, 0.25)])
+def test_geometry_adjoint_is_the_transpose(D, n, jitter):
+    """The adjoint's bars, summed within each cell and then over the cells, are the tangent's transpose for one position at a
+    time and for all together: cell counts around the 64 cells a thread takes at once, a square lattice whose edges meet four at
+    a vertex (a cubic lattice's vertices have no derivative: planes of a vertex are parallel there), and bars added to what
+    xbar held; the same bits every run."""
+    m = mesh.build(problems.jittered_lattice(n, D, jitter, 4), 1.0)
+    g = mesh.GeometryDerivative(m)
+    rng = np.random.default_rng(6)
+    N = m["cells"]
+    bars = [rng.normal(size=s) for s in ((N,), (N, D), (m["faces"], D), (m["faces"], D))]
+    xbar = g.adjoint(*bars)
+    assert np.isfinite(xbar).all()
+    assert np.array_equal(xbar, g.adjoint(*bars))
+    held = rng.normal(size=xbar.shape)
+    # one more rounding of each of the cells' sums (some 17 a position) at the size they have with what was held
+    slack = 17 * 2.0 ** -53 * (np.abs(xbar).max() + np.abs(held).max())
+    assert np.abs(g.adjoint(*bars, xbar=held.copy()) - (held + xbar)).max() <= 17 * slack
+    moves = [rng.normal(size=xbar.shape)]
+    for i in (0, N // 2, N - 1):
+        moves.append(np.zeros(xbar.shape))
+        moves[-1][i] = rng.normal(size=D)
+    for dx in moves:
+        t = g.tangent(dx)
+        lhs = sum(np.sum(b * a) for b, a in zip(bars, t))
+        # some 500 terms a cell, each a vertex's solve whose rows are as short as a tenth of the cell: 500 x 2^-53 x 10
+        scale = sum(np.sum(np.abs(b * a)) for b, a in zip(bars, t)) + np.sum(np.abs(xbar * dx))
+        assert abs(lhs - np.sum(xbar * dx)) < 1e-12 * scale
+    g.close()
