@@ -458,6 +458,13 @@ int sweep(luna_fv* fv, double courant, bool dt_only = false) {
     return LUNA_OK;
 }
 
+// The smallest of a set of dt slots (positive doubles order as their bits).
+double smallest_time_step(const unsigned long long* slots) {
+    unsigned long long least = luna::INF_BITS;
+    for (int k = 0; k < luna::DT_SLOTS; ++k) least = std::min(least, slots[k * luna::DT_STRIDE]);
+    return bits_to_double(least);
+}
+
 // The time step of the sweep that wrote the dt slots of `parity`: their smallest, read back (blocks).
 int read_time_step(luna_fv* fv, int parity, double* dt) {
     unsigned long long* slots = fv->host + 8;
@@ -465,9 +472,7 @@ int read_time_step(luna_fv* fv, int parity, double* dt) {
                             fv->stream));
     LUNA_HIP(hipStreamSynchronize(fv->stream));
     LUNA_HIP(fv->prof.collect());
-    unsigned long long least = luna::INF_BITS;
-    for (int k = 0; k < luna::DT_SLOTS; ++k) least = std::min(least, slots[k * luna::DT_STRIDE]);
-    *dt = bits_to_double(least);
+    *dt = smallest_time_step(slots);
     return LUNA_OK;
 }
 
@@ -1445,7 +1450,10 @@ struct luna_fv1 {
         }
         return a;
     }
-    luna::Counters counters_now() const { return luna::Counters{counters.p + parity, counters.p + (parity ^ 1), counters.p + 2}; }
+    luna::Counters counters_now() const {
+        return luna::Counters{counters.p + parity * luna::DT_WORDS, counters.p + (parity ^ 1) * luna::DT_WORDS, nullptr};
+    }
+    unsigned long long* done() const { return counters.p + 2 * luna::DT_WORDS; }
 };
 
 namespace {
@@ -1493,6 +1501,13 @@ hipError_t reserve_slots(luna_fv1* fv, bool left, bool right) {
     fv->slots = slots;
     fv->lo = lo;
     return hipSuccess;
+}
+
+// A line's counters at its creation: two sets of dt slots, then the arrivals of a watched step.
+std::vector<unsigned long long> line_counters() {
+    std::vector<unsigned long long> init(2 * luna::DT_WORDS + 1, luna::INF_BITS);
+    init.back() = 0;
+    return init;
 }
 
 double host_snap(const luna_fv1* fv, double x) {
@@ -1648,13 +1663,13 @@ int luna_fv1_create(const luna_fv1_options* opt, const luna_line* line, luna_fv1
     const size_t n = fv->n;
     if (hipStreamCreate(&fv->stream) != hipSuccess) return cleanup(fail(LUNA_ERR_DEVICE, "luna: hipStreamCreate failed"));
     if (fv->keys.reserve(n) != hipSuccess || fv->q.reserve(3 * n) != hipSuccess || fv->next.reserve(3 * n) != hipSuccess ||
-        fv->counters.reserve(4) != hipSuccess)
+        fv->counters.reserve(2 * luna::DT_WORDS + 1) != hipSuccess)
         return cleanup(fail(LUNA_ERR_MEMORY, "luna: device allocation failed"));
-    if (hipHostMalloc(reinterpret_cast<void**>(&fv->host), 8 * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess)
+    if (hipHostMalloc(reinterpret_cast<void**>(&fv->host), luna::DT_WORDS * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess)
         return cleanup(fail(LUNA_ERR_MEMORY, "luna: pinned host allocation failed"));
-    const unsigned long long init[4] = {luna::INF_BITS, luna::INF_BITS, 0, 0};
+    const std::vector<unsigned long long> init = line_counters();
     std::vector<double> zero(3 * n, 0.0);
-    if (hipMemcpy(fv->counters.p, init, sizeof init, hipMemcpyHostToDevice) != hipSuccess ||
+    if (hipMemcpy(fv->counters.p, init.data(), sizeof(unsigned long long) * init.size(), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(fv->keys.p, line->keys, sizeof(long long) * n, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(fv->q.p, zero.data(), sizeof(double) * 3 * n, hipMemcpyHostToDevice) != hipSuccess)
         return cleanup(fail(LUNA_ERR_DEVICE, "luna: initial upload failed"));
@@ -1717,16 +1732,17 @@ int luna_fv1_create_moving(const luna_fv1_options* opt, const luna_moving_line* 
     if (fv->q.reserve(3 * static_cast<size_t>(n)) != hipSuccess || fv->next.reserve(3 * static_cast<size_t>(n)) != hipSuccess ||
         fv->x.reserve(n) != hipSuccess || fv->x_next.reserve(n) != hipSuccess || fv->line_key[0].reserve(fv->slots) != hipSuccess ||
         fv->line_key[1].reserve(fv->slots) != hipSuccess || fv->line_id.reserve(fv->slots) != hipSuccess ||
-        fv->counters.reserve(4) != hipSuccess || fv->descents.reserve(2) != hipSuccess || fv->ends.reserve(luna::LINE_ENDS) != hipSuccess ||
+        fv->counters.reserve(2 * luna::DT_WORDS + 1) != hipSuccess || fv->descents.reserve(2) != hipSuccess || fv->ends.reserve(luna::LINE_ENDS) != hipSuccess ||
         fv->inflow_dev.reserve(6) != hipSuccess)
         return cleanup(fail(LUNA_ERR_MEMORY, "luna: device allocation failed"));
     if (hipHostMalloc(reinterpret_cast<void**>(&fv->host), 4 * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc(reinterpret_cast<void**>(&fv->host_ends), luna::LINE_ENDS * sizeof(double), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc(reinterpret_cast<void**>(&fv->host_descents), sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess)
         return cleanup(fail(LUNA_ERR_MEMORY, "luna: pinned host allocation failed"));
-    const unsigned long long init[4] = {luna::INF_BITS, luna::INF_BITS, 0, 0}, zeros[2] = {0, 0};
+    const std::vector<unsigned long long> init = line_counters();
+    const unsigned long long zeros[2] = {0, 0};
     std::vector<double> zero(3 * static_cast<size_t>(n), 0.0);
-    if (hipMemcpy(fv->counters.p, init, sizeof init, hipMemcpyHostToDevice) != hipSuccess ||
+    if (hipMemcpy(fv->counters.p, init.data(), sizeof(unsigned long long) * init.size(), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(fv->descents.p, zeros, sizeof zeros, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(fv->line_key[0].p, key.data(), sizeof(long long) * fv->slots, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(fv->line_id.p, id.data(), sizeof(int) * fv->slots, hipMemcpyHostToDevice) != hipSuccess ||
@@ -1830,7 +1846,7 @@ int luna_fv1_time_step(luna_fv1* fv, double courant, int rule, double* dt) {
     const int slot = fv->parity;
     LUNA_HIP(luna::launch_line_time_step(fv->stream, fv->args(), courant, rule == LUNA_STEP_LUNA, fv->counters_now()));
     fv->parity ^= 1;
-    LUNA_HIP(hipMemcpyAsync(fv->host, fv->counters.p + slot, sizeof(unsigned long long), hipMemcpyDeviceToHost, fv->stream));
+    LUNA_HIP(hipMemcpyAsync(fv->host, fv->counters.p + slot * luna::DT_WORDS, sizeof(unsigned long long), hipMemcpyDeviceToHost, fv->stream));
     if (fv->moving && fv->watching) {
         // finite_volume_1d.hpp:372-381: while gas enters, what the end slots ask their walls for
         const int rc = read_ends(fv);
@@ -1846,7 +1862,7 @@ int luna_fv1_time_step(luna_fv1* fv, double courant, int rule, double* dt) {
 int luna_fv1_step(luna_fv1* fv, double dt) {
     if (!fv) return fail(LUNA_ERR_ARGUMENT, "luna_fv1_step: null argument");
     if (!fv->moving) {
-        LUNA_HIP(luna::launch_line_step(fv->stream, fv->args(), dt, 0.0, false, fv->counters_now(), fv->counters.p + 2, fv->host));
+        LUNA_HIP(luna::launch_line_step(fv->stream, fv->args(), dt, 0.0, false, fv->counters_now(), fv->done(), fv->host));
         std::swap(fv->q, fv->next);
         return LUNA_OK;
     }
@@ -1902,7 +1918,7 @@ int luna_fv1_step_and_time_step(luna_fv1* fv, double dt, double courant, double*
         unsigned long long descents = 0;
         if ((rc = moving_kernel(fv, dt, courant, true, &descents)) != LUNA_OK) return rc;
         fv->parity ^= 1;
-        LUNA_HIP(hipMemcpyAsync(fv->host, fv->counters.p + slot, sizeof(unsigned long long), hipMemcpyDeviceToHost, fv->stream));
+        LUNA_HIP(hipMemcpyAsync(fv->host, fv->counters.p + slot * luna::DT_WORDS, sizeof(unsigned long long), hipMemcpyDeviceToHost, fv->stream));
         LUNA_HIP(hipStreamSynchronize(fv->stream));
         *next = bits_to_double(fv->host[0]);
         bool again = false, added = false;
@@ -1918,11 +1934,18 @@ int luna_fv1_step_and_time_step(luna_fv1* fv, double dt, double courant, double*
         return LUNA_OK;
     }
     fv->host[0] = LINE_NO_STEP;
-    LUNA_HIP(luna::launch_line_step(fv->stream, fv->args(), dt, courant, true, fv->counters_now(), fv->counters.p + 2, fv->host));
+    LUNA_HIP(luna::launch_line_step(fv->stream, fv->args(), dt, courant, true, fv->counters_now(), fv->done(), fv->host));
     fv->parity ^= 1;
     std::swap(fv->q, fv->next);
-    if (int rc = await_line_step(fv)) return rc;
-    *next = bits_to_double(fv->host[0]);
+    if (luna::line_watched(fv->n)) {
+        if (int rc = await_line_step(fv)) return rc;
+        *next = bits_to_double(fv->host[0]);
+        return LUNA_OK;
+    }
+    LUNA_HIP(hipMemcpyAsync(fv->host, fv->counters.p + slot * luna::DT_WORDS, sizeof(unsigned long long) * luna::DT_WORDS, hipMemcpyDeviceToHost,
+                            fv->stream));
+    LUNA_HIP(hipStreamSynchronize(fv->stream));
+    *next = smallest_time_step(fv->host);
     return LUNA_OK;
 }
 

@@ -115,7 +115,8 @@ struct Grid {
 
 // The mesh sweeps' min-reduction goes to DT_SLOTS addresses a cache line apart (work-group b to slot b mod DT_SLOTS), whose
 // smallest the host takes: atomics to one address are served one after the other, about 11 ns each on MI355X, so that the
-// 4096 wavefronts of a 511^2 sweep took 76 us with one address and take 38 with 32. (A line's kernels use the first alone.)
+// 4096 wavefronts of a 511^2 sweep took 76 us with one address and take 38 with 32. (A line's kernels use the first alone,
+// but for the static step of a long line.)
 constexpr int DT_SLOTS = 32, DT_STRIDE = 16, DT_WORDS = DT_SLOTS * DT_STRIDE;
 struct Counters {
     unsigned long long* dt;         // the min-reduction this sweep writes
@@ -254,8 +255,15 @@ struct LineArgs {
     long long* key_next;  // by slot: the key of the slot's point after the step
 };
 hipError_t launch_line_time_step(hipStream_t s, const LineArgs& a, double courant, int luna_rule, const Counters& c);
-// The static step; fused, also the next dt by LUNA's rule into c.dt and, when the kernel is done, into *host (pinned host
-// memory). done: a word of device memory that is zero between launches.
+// The static step; fused, also the next dt by LUNA's rule: of a line that is watched into c.dt and, when the kernel is done,
+// into *host (pinned host memory), else into the DT_SLOTS words of c.dt. done: a word of device memory that is zero between
+// launches.
+// Where the line lies: a watched line's wavefronts make two atomics each on one line of memory, served one after the other,
+// 17 us a fused step at 16384 cells, 22 at 32768, 130 at 262144 and 508 at a million; the copy of DT_SLOTS words and the wait
+// for the stream cost 19 us up to 32768 cells, 25 at 262144 and 47 at a million (the kernel with one atomic per 256 cells of
+// five-cell stencils: 25, 25, 37 and 88 us).
+constexpr int LINE_WATCHED_MAX = 16384;
+inline bool line_watched(int cells) { return cells <= LINE_WATCHED_MAX; }
 hipError_t launch_line_step(hipStream_t s, const LineArgs& a, double dt, double courant, bool fused, const Counters& c,
                             unsigned long long* done, unsigned long long* host);
 // The moving step: Q, positions and keys after the step into a.next, a.x_next, a.key_next; the count of adjacent slots

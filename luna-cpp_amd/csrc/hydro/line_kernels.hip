@@ -20,15 +20,16 @@ __device__ __forceinline__ double wave_min(double v) {
     for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o));
     return v;
 }
+template <int B = BLOCK>
 __device__ __forceinline__ void block_min(double v, unsigned long long* out) {
-    __shared__ double part[BLOCK / 64];
+    __shared__ double part[B / 64];
     v = wave_min(v);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (lane == 0) part[wave] = v;
     __syncthreads();
     if (threadIdx.x == 0) {
         double m = part[0];
-        for (int k = 1; k < (int)(blockDim.x >> 6); ++k) m = fmin(m, part[k]);
+        for (int k = 1; k < B / 64; ++k) m = fmin(m, part[k]);
         if (m < INFINITY) atomicMin(out, (unsigned long long)__double_as_longlong(m));
     }
 }
@@ -434,20 +435,29 @@ __global__ void k_line_unpack(const unsigned long long* packed, int n, long long
     }
 }
 
+// The other set of time-step words, reset for the next sweep, in whichever way that one reduces.
+__device__ __forceinline__ void reset_next(unsigned long long* dt_next) {
+    if (blockIdx.x == 0 && threadIdx.x < DT_SLOTS) dt_next[threadIdx.x * DT_STRIDE] = INF_BITS;
+}
+
 // One static step (finite_volume_1d.hpp:389-407, 555-600): a wavefront takes LINE_OUT consecutive slots and two more at each
 // end; lane t holds slot first + t - 2. Each lane computes its own cell's primitives, limited gradient and two face states
 // and the flux of its right face once, and takes its neighbours' by shuffles. What bounds it is the length of that chain
 // (a line of 1024 cells fills 18 wavefronts of the chip): with the five-cell stencil, three gradients and two fluxes
 // computed by every work-item the kernel took 12.0 us at 1024 cells, now 6.2.
+// Fused, WAVES = 1: every wavefront's minimum and arrival go to one word each and the last to arrive hands the minimum to
+// the host. WAVES = 4 (a long line, where those atomics would be the step's time): one minimum per work-group, spread over
+// DT_SLOTS words that the host reads when the stream is done.
 constexpr int LINE_OUT = 60;
 __device__ __forceinline__ void from_lane(const double* v, int lane, double* out) {
 #pragma unroll
     for (int k = 0; k < 3; ++k) out[k] = __shfl(v[k], lane);
 }
-__global__ __launch_bounds__(64) void k_line_step(LineArgs l, double dt, double courant, int fused, unsigned long long* dt_out,
-                                                  unsigned long long* dt_next, unsigned long long* done, unsigned long long* host) {
-    const int lane = threadIdx.x, s = blockIdx.x * LINE_OUT + lane - 2;
-    if (blockIdx.x == 0 && lane == 0 && fused) *dt_next = INF_BITS;
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void k_line_step(LineArgs l, double dt, double courant, int fused, unsigned long long* dt_out,
+                                                          unsigned long long* dt_next, unsigned long long* done, unsigned long long* host) {
+    const int lane = threadIdx.x & 63, s = (blockIdx.x * WAVES + (threadIdx.x >> 6)) * LINE_OUT + lane - 2;
+    if (fused) reset_next(dt_next);
     const int t = slot(l, s, 0);  // -1 past a wall
     const bool real = t >= 0;
     Cell cell[3] = {};  // the left neighbour's, this lane's, the right neighbour's
@@ -513,7 +523,8 @@ __global__ __launch_bounds__(64) void k_line_step(LineArgs l, double dt, double 
             smallest = courant * me.V / (fabs(Wn[1]) + sound_speed<1>(l.gas, Wn));
         }
     }
-    if (fused) {
+    if (!fused) return;
+    if constexpr (WAVES == 1) {
         smallest = wave_min(smallest);
         if (lane == 0) {
             if (smallest < INFINITY) atomicMin(dt_out, (unsigned long long)__double_as_longlong(smallest));
@@ -526,6 +537,8 @@ __global__ __launch_bounds__(64) void k_line_step(LineArgs l, double dt, double 
                 __hip_atomic_store(host, atomicMin(dt_out, INF_BITS), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
             }
         }
+    } else {
+        block_min<64 * WAVES>(smallest, dt_out + (blockIdx.x % DT_SLOTS) * DT_STRIDE);
     }
 }
 
@@ -533,7 +546,7 @@ __global__ __launch_bounds__(64) void k_line_step(LineArgs l, double dt, double 
 __global__ __launch_bounds__(BLOCK) void k_line_time_step(LineArgs l, double courant, int luna_rule, unsigned long long* dt_out,
                                                           unsigned long long* dt_next) {
     const int s = blockIdx.x * BLOCK + threadIdx.x;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *dt_next = INF_BITS;
+    reset_next(dt_next);
     double smallest = INFINITY;
     if (s < l.n) {
         double Wi[3];
@@ -934,8 +947,11 @@ hipError_t launch_line_time_step(hipStream_t s, const LineArgs& a, double couran
 
 hipError_t launch_line_step(hipStream_t s, const LineArgs& a, double dt, double courant, bool fused, const Counters& c,
                             unsigned long long* done, unsigned long long* host) {
-    hipLaunchKernelGGL(k_line_step, dim3((a.n + LINE_OUT - 1) / LINE_OUT), dim3(64), 0, s, a, dt, courant, fused ? 1 : 0, c.dt, c.dt_next,
-                       done, host);
+    const int waves = (a.n + LINE_OUT - 1) / LINE_OUT;
+    if (line_watched(a.n))
+        hipLaunchKernelGGL(k_line_step<1>, dim3(waves), dim3(64), 0, s, a, dt, courant, fused ? 1 : 0, c.dt, c.dt_next, done, host);
+    else
+        hipLaunchKernelGGL(k_line_step<4>, dim3((waves + 3) / 4), dim3(256), 0, s, a, dt, courant, fused ? 1 : 0, c.dt, c.dt_next, done, host);
     return hipGetLastError();
 }
 
