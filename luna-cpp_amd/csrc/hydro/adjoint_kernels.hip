@@ -6,6 +6,7 @@
 #include <type_traits>
 
 #include "derivatives.hpp"
+#include "fit.hpp"
 #include "kernels.hpp"
 #include "staged.hpp"
 
@@ -59,37 +60,6 @@ struct Pattern {
 template <int D>
 __device__ __forceinline__ double bound_tangent(const Geo& g, int base, const Pattern<D>& pat, int v, const double* dW) {
     return pat.extreme[v] < 0 ? 0.0 : dW[(size_t)g.other[base + pat.extreme[v] * SLICE] * (D + 2) + v];
-}
-
-// M x = b of the fit with its Cholesky factor L, in the sweep's operation order. Fast: with the correctly rounded quotients of
-// exact_math.hpp by L's diagonal (by), the same bits for operands in their range.
-template <int D, bool Fast>
-__device__ __forceinline__ void solve_fit(const double (*L)[D + 1], const Divisor* by, const double* b, double* x) {
-    constexpr int U = D + 1;
-    double z[U];
-#pragma unroll
-    for (int p = 0; p < U; ++p) {
-        double sum = b[p];
-#pragma unroll
-        for (int m = 0; m < p; ++m) sum -= L[p][m] * z[m];
-        z[p] = Fast ? over(sum, by[p]) : sum / L[p][p];
-    }
-#pragma unroll
-    for (int p = U - 1; p >= 0; --p) {
-        double sum = z[p];
-#pragma unroll
-        for (int m = p + 1; m < U; ++m) sum -= L[m][p] * x[m];
-        x[p] = Fast ? over(sum, by[p]) : sum / L[p][p];
-    }
-}
-// Whether solves with this factor and right-hand sides of absolute sum `size` stay in the fast quotients' range: diagonals
-// within 2^200 of 1 and a size under 2^200 bound every quotient on the way by 2^1000.
-template <int D>
-__device__ __forceinline__ bool solves_fast(const double (*L)[D + 1], double size) {
-    bool ok = size < 0x1p200;
-#pragma unroll
-    for (int p = 0; p <= D; ++p) ok = ok && L[p][p] > 0x1p-200 && L[p][p] < 0x1p200;
-    return ok;
 }
 
 // The cell's fit and limiter as the sweep computes them (the same bits for g), with the unlimited gradient g0, its tangent
@@ -191,36 +161,35 @@ __device__ void fit_cell(const Geo& g, int i, const double* dW, bool limit, doub
             for (int m = 0; m < q; ++m) sum -= L[p][m] * L[q][m];
             L[p][q] = p == q ? sqrt(sum) : sum / L[q][q];
         }
-    double size = 0;
 #pragma unroll
     for (int p = 0; p < U; ++p) M0[p] = M[0][p];
+    Divisor by[U];
+    FitRange range;
 #pragma unroll
-    for (int v = 0; v < V; ++v)
-#pragma unroll
-        for (int p = 0; p < U; ++p) size += fabs(b[v][p]) + (Tangent ? fabs(db[v][p]) : 0.0);
-    const auto solve = [&](auto fast) {
-        constexpr bool Fast = decltype(fast)::value;
-        Divisor by[U];
-#pragma unroll
-        for (int p = 0; p < U; ++p) by[p] = Fast ? divisor(L[p][p]) : Divisor{L[p][p], 0.0};
+    for (int p = 0; p < U; ++p) {
+        by[p] = divisor(L[p][p]);
+        range.divisor.large(L[p][p]);
+        range.divisor.small(L[p][p]);
+    }
+    double x[V][U], dx[V][U];
+    const auto solve_all = [&](auto fast) {
 #pragma unroll
         for (int v = 0; v < V; ++v) {
-            double x[U];
-            solve_fit<D, Fast>(L, by, b[v], x);
-#pragma unroll
-            for (int a = 0; a < D; ++a) g0[v * D + a] = gl[v * D + a] = x[1 + a];
-            if (intercept) intercept[v] = x[0];
-            if constexpr (Tangent) {
-                solve_fit<D, Fast>(L, by, db[v], x);
-#pragma unroll
-                for (int a = 0; a < D; ++a) dg0[v * D + a] = x[1 + a];
-            }
+            solve<D, decltype(fast)::value>(L, by, b[v], x[v], range);
+            if constexpr (Tangent) solve<D, decltype(fast)::value>(L, by, db[v], dx[v], range);
         }
     };
-    if (__all(solves_fast<D>(L, size)))
-        solve(std::true_type{});
-    else
-        solve(std::false_type{});
+    solve_all(std::true_type{});
+    if (!__all(range.ok())) solve_all(std::false_type{});
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            g0[v * D + a] = gl[v * D + a] = x[v][1 + a];
+            if constexpr (Tangent) dg0[v * D + a] = dx[v][1 + a];
+        }
+        if (intercept) intercept[v] = x[v][0];
+    }
 #pragma unroll
     for (int v = 0; v < V; ++v) {
         pat.last[v] = -1;

@@ -184,6 +184,7 @@ struct luna_fv {
     Buf<long long> geo_info;
     Buf<unsigned int> geo_flags;
     bool mesh_ok = false;  // the last mesh given was accepted
+    bool far_offsets = false;
     // The accepted mesh's arrays: the step reads its face arrays in place (a device mesh's, or the copies of a host mesh in
     // the src_ buffers); `records` once the derivatives' face records are built for it.
     luna::MeshIn mesh{};
@@ -206,6 +207,7 @@ struct luna_fv {
         g.fcen = mesh.face_centroid;
         g.slot = slotgeo.p;
         g.slots = slots;
+        g.far_offsets = far_offsets;
         for (int a = 0; a < 3; ++a) {
             g.side[a] = side[a];
             g.inverse[a] = side[a] > 0 ? 1.0 / side[a] : 0.0;
@@ -300,6 +302,7 @@ int derive(luna_fv* fv, const luna_geometry* m, luna::MeshIn in, bool eager_reco
     flags = static_cast<unsigned int>(back[1]);
     if (flags & luna::GEO_BAD_CELL) return fail(LUNA_ERR_ARGUMENT, "luna: face cell index out of range");
     if (flags & luna::GEO_BAD_FACE) return fail(LUNA_ERR_ARGUMENT, "luna: list entry out of range or not a face of its cell");
+    fv->far_offsets = (flags & luna::GEO_FAR_OFFSETS) != 0;
     fv->F = F;
     fv->E = 2 * F;
     fv->slots = static_cast<int>(slots);

@@ -247,7 +247,10 @@ __global__ __launch_bounds__(SLOT_BLOCK) void k_geo_slots(MeshIn m, const int* _
                     }
                 }
 #pragma unroll
-                for (int a = 0; a < D; ++a) off[a] = rel[a] - s_cen[lane * D + a];
+                for (int a = 0; a < D; ++a) {
+                    off[a] = rel[a] - s_cen[lane * D + a];
+                    if (!(fabs(off[a]) < FAR_OFFSET)) bad |= GEO_FAR_OFFSETS;
+                }
             }
         }
         if (t < QUARTER_DEPTH) {

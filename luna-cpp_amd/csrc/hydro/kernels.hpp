@@ -55,6 +55,7 @@ struct Geo {
     // to this cell's centroid (Geometry::face_offset, finite_volume.hpp:322-326), one plane per axis
     const double* slot;
     long long slots;
+    bool far_offsets;            // some face offset is FAR_OFFSET or more (GEO_FAR_OFFSETS)
     double side[3], inverse[3];  // the periodic box and 1 / side
 };
 
@@ -75,6 +76,10 @@ struct MeshIn {
 };
 // Flags the geometry pass raises on a malformed mesh (it then reads nothing out of range and the host refuses the mesh).
 constexpr unsigned int GEO_BAD_START = 1, GEO_BAD_CELL = 2, GEO_BAD_FACE = 4, GEO_TOO_MANY_SLOTS = 8;
+// Not a fault: a face offset of 2^105 or more, infinite or NaN. The limiter's changes there may leave the range of the fast
+// quotients.
+constexpr unsigned int GEO_FAR_OFFSETS = 16;
+constexpr double FAR_OFFSET = 0x1p105;
 
 // Per-cell rows of the step (device pointers).
 struct Rows {

@@ -11,6 +11,7 @@
 #include <type_traits>
 
 #include "exact_math.hpp"
+#include "fit.hpp"
 #include "kernels.hpp"
 #include "staged.hpp"
 
@@ -22,7 +23,10 @@
 #ifndef LUNA_UPDATE_UNROLL
 #define LUNA_UPDATE_UNROLL 4
 #endif
-#ifndef LUNA_SWEEP_WAVES  // 2 (178 and 188 VGPRs, no spill): 0.72 ms static and 0.44 ms moving; 3 spills 32 to 120 B: 0.74 and 0.74
+// 2 (178 and 192 VGPRs, no spill): 0.72 ms static at 128^3 and 0.44 ms moving at 104^3; 3 spills 32 to 120 B: 0.74 ms at each.
+// The reduced-precision sweeps take 3 (168 VGPRs, up to 20 B spilled): at 72^3 0.125 ms static and 0.147 moving, against 0.144
+// and 0.157 with 2.
+#ifndef LUNA_SWEEP_WAVES
 #define LUNA_SWEEP_WAVES 2
 #endif
 #ifndef LUNA_FLUX_WAVES
@@ -257,17 +261,17 @@ __device__ __forceinline__ float lower(float a, float b) { return fminf(a, b); }
 __device__ __forceinline__ float higher(float a, float b) { return fmaxf(a, b); }
 
 // The sweep's per-cell sums (finite_volume.hpp:486-515), in list order. G: the fit's type (double, or float for the
-// reduced-precision policies, whose range is of W_j - W_i, rounded once, :466-469, 510-512). Fast: ok tells whether every
-// operand was in the range of the fast operators.
-template <int D, bool Moving, bool Grad, int Rule, class G = double, bool Fast = false>
+// reduced-precision policies, whose range is of W_j - W_i, rounded once, :466-469, 510-512). operands: the range of what
+// add<true>() divides by or takes the root of.
+template <int D, bool Moving, bool Grad, int Rule, class G = double>
 struct Sums {
     static constexpr int V = D + 2, U = D + 1;
     static constexpr bool exact = sizeof(G) == 8;
-    using Op = Arith<Fast>;
     double max_angle = 0, smallest = INFINITY;
     G lo[V], hi[V], M[U][U], b[V][U];
-    bool ok = true;
+    Range operands;
 
+    __device__ __forceinline__ bool ok() const { return operands.within(500, 501); }
     __device__ __forceinline__ void init_range() {
 #pragma unroll
         for (int v = 0; v < V; ++v) {
@@ -295,17 +299,23 @@ struct Sums {
             hi[v] = higher(hi[v], value);
         }
     }
+    template <bool Fast>
     __device__ __forceinline__ void add(const Geo& g, const Near<D>& n, const double* xi, const double* centroid, const double* Wi,
                                         double csi, double ri, double courant, double tiny) {
+        using Op = Arith<Fast>;
         double d[D];
         separation<D>(g, xi, n.x, d);
         const double magnitude = n.mag;
         const double dd = dot<D>(d, d), dist = Op::square_root(dd);
         const Divisor by_dist = Op::by(dist);
-        if constexpr (Fast) ok = ok && plain(dd);
+        if constexpr (Fast) {
+            operands.small(dd);
+            operands.large(dd);
+        }
         if constexpr (Moving) {
+            if constexpr (Fast) operands.large(magnitude);
             if constexpr (Fast && D == 3) {  // face_angle<3>: 1 / pi rounded to nearest, as divisor() would give it
-                ok = ok && plain(magnitude);
+                operands.small(magnitude);
                 const double angle = root(over(magnitude, Divisor{M_PI, M_1_PI}));
                 max_angle = higher(max_angle, over(angle, Divisor{0.5 * dist, 2.0 * by_dist.y}));
             } else {
@@ -334,8 +344,12 @@ struct Sums {
             double dv[D];
 #pragma unroll
             for (int a = 0; a < D; ++a) dv[a] = n.W[1 + a] - Wi[1 + a];
+            // (a dv . d too small for the quotient's last bit is too small for vsig's, which is in range)
             const double vsig = csi + n.cs - Op::quotient(dot<D>(dv, d), by_dist);
-            if constexpr (Fast) ok = ok && plain(vsig);
+            if constexpr (Fast) {
+                operands.small(fabs(vsig));
+                operands.large(vsig);
+            }
             const double term = courant * Op::quotient(dist + ri, Op::by(vsig));
             smallest = vsig > 0 && term < smallest ? term : smallest;
         }
@@ -351,16 +365,51 @@ struct Sums {
 // row loads an entry) and the limiter a third. Measured at 128^3 (waves in every variable and a blast), static: 0.95 ms with
 // rows loaded lane by lane, the compiler's divisions, the range walked again for tiny faces and the clips in branches; 0.79
 // with the surface summed first, the fast operators and the clips side by side; 0.72 with the rows through LDS. Moving, 104^3:
-// 0.63, 0.62, 0.44 ms. One wavefront, a slice of 64 cells; Fast as Arith: returns false, having written
-// nothing, if some operand of the wavefront was out of the fast operators' range. smallest: the smallest time-step term.
-template <int D, bool Moving, bool Grad, int Limit, int Rule, int Prec, bool Fast>
-__device__ __forceinline__ bool sweep_slice(const Geo& g, const Rows& r, double courant, int block, lds_double* lds, double& smallest) {
+// 0.63, 0.62, 0.44 ms. One wavefront, a slice of 64 cells; the walk of its lists, with the operators of Fast, tells whether
+// their operands were in range for all 64.
+template <bool Fast, int D, class S>
+__device__ __forceinline__ bool walk_lists(const Geo& g, const double* xi, const double* centroid, const double* Wi, double ci, double ri,
+                                           double courant, double tiny, int count, int depth, const int* other, const double* geometry, int lane,
+                                           lds_double* lds, S& s) {
+    s.init();
+    // While entry t is summed, the rows of entry t + 1 are on their way to LDS and those of entry t + 2 asked for. Every lane
+    // takes part in every fetch; the list's padding names cell 0, and past the end the last entry is fetched again, so that
+    // two fetches are always in flight.
+    Stage<D> stage;
+    stage.init(lane, lds);
+    const int last = depth - 1;
+    if (depth > 0) {
+        int next = (other + min(2, last) * SLICE)[lane];
+        stage.address(other[lane]);
+        stage.fetch(g.cell, 0);
+        stage.address((other + min(1, last) * SLICE)[lane]);
+        stage.fetch(g.cell, 1);
+        double mag = geometry[lane];
+        stage.address(next);
+        next = (other + min(3, last) * SLICE)[lane];
+        for (int t = 0; t < depth; ++t) {
+            Near<D> n;
+            stage.read(t & 1, n);
+            n.mag = mag;
+            mag = (geometry + min(t + 1, last) * SLICE)[lane];
+            const int after = (other + min(t + 4, last) * SLICE)[lane];
+            stage.fetch(g.cell, t & 1);  // the last loads of the iteration: read() counts on it
+            stage.address(next);
+            next = after;
+            if (t < count) s.template add<Fast>(g, n, xi, centroid, Wi, ci, ri, courant, tiny);
+        }
+        stage.drain();
+    }
+    return __all(s.ok());
+}
+
+template <int D, bool Moving, bool Grad, int Limit, int Rule, int Prec>
+__device__ __forceinline__ void sweep_slice(const Geo& g, const Rows& r, double courant, int block, lds_double* lds, double& smallest) {
     constexpr int V = D + 2, U = D + 1;
     using G = typename std::conditional<Prec == 0, double, float>::type;
     constexpr bool exact = Prec == 0;
     static_assert(exact || Limit < 2, "the learned limiter's features need the double policy");
     using C = CellAt<D>;
-    using Op = Arith<Fast && exact>;
     const unsigned lane = threadIdx.x;
     const int i = block * CELL_BLOCK + (int)lane;
     const bool here = i < g.N;
@@ -371,8 +420,6 @@ __device__ __forceinline__ bool sweep_slice(const Geo& g, const Rows& r, double 
     const double ci = mine[C::CS], ri = mine[C::RAD];
     load_vec<D>(mine + C::X, xi);
     load_vec<D>(mine + C::C, centroid);
-    Sums<D, Moving, Grad, Rule, G, Fast> s;
-    s.init();
     const int first = g.slice[block];
     const int* other = g.other + first;       // the slice's entries: entry t of lane l at t SLICE + l
     const double* geometry = g.slot + first;  // |A|; the face offsets a + 1 times g.slots further
@@ -392,89 +439,65 @@ __device__ __forceinline__ bool sweep_slice(const Geo& g, const Rows& r, double 
         }
         tiny = 1e-6 * surface;
     }
-    {
-        // The list walk: while entry t is summed, the rows of entry t + 1 are on their way to LDS and those of entry t + 2
-        // asked for. Every lane takes part in every fetch; the list's padding names cell 0, and past the end the last
-        // entry is fetched again, so that two fetches are always in flight.
-        Stage<D> stage;
-        stage.init(lane, lds);
-        const int last = depth - 1;
-        if (depth > 0) {
-            int next = (other + min(2, last) * SLICE)[lane];
-            stage.address(other[lane]);
-            stage.fetch(g.cell, 0);
-            stage.address((other + min(1, last) * SLICE)[lane]);
-            stage.fetch(g.cell, 1);
-            double mag = geometry[lane];
-            stage.address(next);
-            next = (other + min(3, last) * SLICE)[lane];
-            for (int t = 0; t < depth; ++t) {
-                Near<D> n;
-                stage.read(t & 1, n);
-                n.mag = mag;
-                mag = (geometry + min(t + 1, last) * SLICE)[lane];
-                const int after = (other + min(t + 4, last) * SLICE)[lane];
-                stage.fetch(g.cell, t & 1);  // the last loads of the iteration: read() counts on it
-                stage.address(next);
-                next = after;
-                if (t < count) s.add(g, n, xi, centroid, Wi, ci, ri, courant, tiny);
-            }
-            stage.drain();
-        }
-    }
+    Sums<D, Moving, Grad, Rule, G> s;
+    if (!walk_lists<true, D>(g, xi, centroid, Wi, ci, ri, courant, tiny, count, depth, other, geometry, lane, lds, s))
+        walk_lists<false, D>(g, xi, centroid, Wi, ci, ri, courant, tiny, count, depth, other, geometry, lane, lds, s);
     smallest = s.smallest;
-    bool ok = s.ok;
     G grad[V][D], intercept[V];
+    [[maybe_unused]] bool fast = true;
     if constexpr (Grad) {  // Sweep::solve (:590-615): Cholesky of M, then M x = b per variable
         G L[U][U];
-        Divisor by[U];
+        if constexpr (exact) {
+            Divisor by[U];
+            double x[V][U];
+            FitRange range;
+            factor<D, true>(s.M, L, by, range);
 #pragma unroll
-        for (int p = 0; p < U; ++p)
+            for (int v = 0; v < V; ++v) solve<D, true>(L, by, s.b[v], x[v], range);
+            fast = __all(range.ok() || !here);
+            if (!fast) {
+                factor<D, false>(s.M, L, by, range);
 #pragma unroll
-            for (int q = 0; q <= p; ++q) {
-                G sum = s.M[q][p];
+                for (int v = 0; v < V; ++v) solve<D, false>(L, by, s.b[v], x[v], range);
+            }
 #pragma unroll
-                for (int m = 0; m < q; ++m) sum -= L[p][m] * L[q][m];
-                if constexpr (exact) {
-                    L[p][q] = p == q ? Op::square_root(sum) : Op::quotient(sum, by[q]);
-                    if (p == q) {
-                        by[p] = Op::by(L[p][p]);
-                        if constexpr (Fast) ok = ok && plain(L[p][p]);
-                    }
-                } else {
+            for (int v = 0; v < V; ++v) {
+#pragma unroll
+                for (int a = 0; a < D; ++a) grad[v][a] = x[v][1 + a];
+                intercept[v] = x[v][0];
+            }
+        } else {
+#pragma unroll
+            for (int p = 0; p < U; ++p)
+#pragma unroll
+                for (int q = 0; q <= p; ++q) {
+                    G sum = s.M[q][p];
+#pragma unroll
+                    for (int m = 0; m < q; ++m) sum -= L[p][m] * L[q][m];
                     L[p][q] = p == q ? sqrt(sum) : sum / L[q][q];
                 }
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                G z[U], x[U];
+#pragma unroll
+                for (int p = 0; p < U; ++p) {
+                    G sum = s.b[v][p];
+#pragma unroll
+                    for (int m = 0; m < p; ++m) sum -= L[p][m] * z[m];
+                    z[p] = sum / L[p][p];
+                }
+#pragma unroll
+                for (int p = U - 1; p >= 0; --p) {
+                    G sum = z[p];
+#pragma unroll
+                    for (int m = p + 1; m < U; ++m) sum -= L[m][p] * x[m];
+                    x[p] = sum / L[p][p];
+                }
+#pragma unroll
+                for (int a = 0; a < D; ++a) grad[v][a] = x[1 + a];
+                intercept[v] = x[0];
             }
-        auto divide = [&](G a, int p) -> G {
-            if constexpr (exact)
-                return Op::quotient(a, by[p]);
-            else
-                return a / L[p][p];
-        };
-        G size = 0;
-#pragma unroll
-        for (int v = 0; v < V; ++v) {
-            G z[U], x[U];
-#pragma unroll
-            for (int p = 0; p < U; ++p) {
-                G sum = s.b[v][p];
-#pragma unroll
-                for (int m = 0; m < p; ++m) sum -= L[p][m] * z[m];
-                z[p] = divide(sum, p);
-            }
-#pragma unroll
-            for (int p = U - 1; p >= 0; --p) {
-                G sum = z[p];
-#pragma unroll
-                for (int m = p + 1; m < U; ++m) sum -= L[m][p] * x[m];
-                x[p] = divide(sum, p);
-                if constexpr (Fast && exact) size += fabs(x[p]);
-            }
-#pragma unroll
-            for (int a = 0; a < D; ++a) grad[v][a] = x[1 + a];
-            intercept[v] = x[0];
         }
-        if constexpr (Fast && exact) ok = ok && size < 0x1p900;  // an overflow on the way leaves a NaN in some x
     }
     double wi[D];
 #pragma unroll
@@ -510,82 +533,90 @@ __device__ __forceinline__ bool sweep_slice(const Geo& g, const Rows& r, double 
     }
     [[maybe_unused]] Record<D, Limit == 2> rec;
     if constexpr (Grad && Limit > 0) {  // the face-centroid limiter, face by face in list order (:538-565)
-        if constexpr (Fast && exact) {  // the rooms the clips divide by the change: none too small for over()
+        if constexpr (exact) {
+            // The rooms the clips divide by the change: none too small for over(). A change beyond its room is at least
+            // about as large, and below 2^DIVISOR_MOST by FitRange's size and the mesh's offsets.
+            Range rooms;
 #pragma unroll
             for (int v = 0; v < V; ++v) {
-                const double up = s.hi[v] - Wi[v], down = Wi[v] - s.lo[v];
-                ok = ok && (!(up > 0) || up > 0x1p-900) && (!(down > 0) || down > 0x1p-900);
+                rooms.small_or_zero(s.hi[v] - Wi[v]);
+                rooms.small_or_zero(s.lo[v] - Wi[v]);
             }
+            fast = fast && !g.far_offsets && __all(rooms.exponent > -NUMERATOR || !here);
+            rec.init(grad);
         }
         // Geometry::face_offset (:322-326), kept per slot, of UL entries loaded together, then applied in order. A face
         // clips the variables it must in one pass over all of them without branches (a factor of 1 leaves a gradient as it
         // is), so their divisions run side by side.
         constexpr int UL = LUNA_LIMIT_UNROLL;
-        if constexpr (exact) rec.init(grad);
-        for (int t0 = 0; t0 < depth; t0 += UL) {
-            double offset[UL][D], mag[UL];
+        const auto limit = [&](auto quick) {
+            using Op = Arith<decltype(quick)::value>;
+            for (int t0 = 0; t0 < depth; t0 += UL) {
+                double offset[UL][D], mag[UL];
 #pragma unroll
-            for (int u = 0; u < UL; ++u) {
-                const double* entry = geometry + min(t0 + u, depth - 1) * SLICE;
-                mag[u] = entry[lane];
+                for (int u = 0; u < UL; ++u) {
+                    const double* entry = geometry + min(t0 + u, depth - 1) * SLICE;
+                    mag[u] = entry[lane];
 #pragma unroll
-                for (int a = 0; a < D; ++a) offset[u][a] = (entry + (a + 1) * g.slots)[lane];
-            }
+                    for (int a = 0; a < D; ++a) offset[u][a] = (entry + (a + 1) * g.slots)[lane];
+                }
 #pragma unroll
-            for (int u = 0; u < UL; ++u) {
-                const bool use = t0 + u < count && !(mag[u] < tiny);
-                if constexpr (exact) {
-                    double dp[V], bound[V];
-                    bool clip[V], any = false;
-#pragma unroll
-                    for (int v = 0; v < V; ++v) {
-                        dp[v] = dot<D>(grad[v], offset[u]);
-                        const double at = Wi[v] + dp[v];
-                        const bool up = dp[v] > 0 && at > s.hi[v], down = dp[v] < 0 && at < s.lo[v];
-                        clip[v] = use && (up || down);
-                        bound[v] = dp[v] > 0 ? s.hi[v] : s.lo[v];
-                        any = any || clip[v];
-                    }
-                    if (use) rec.face(offset[u]);
-                    if (__any(any)) {
+                for (int u = 0; u < UL; ++u) {
+                    const bool use = t0 + u < count && !(mag[u] < tiny);
+                    if constexpr (exact) {
+                        double dp[V], bound[V];
+                        bool clip[V], any = false;
 #pragma unroll
                         for (int v = 0; v < V; ++v) {
-                            // (bound - W) / dp where the bound is on the change's side of W, else 0
-                            const double q = Op::quotient(bound[v] - Wi[v], Op::by(dp[v]));
-                            const double sc = clip[v] ? (q > 0 ? q : 0.0) : 1.0;
-#pragma unroll
-                            for (int a = 0; a < D; ++a) grad[v][a] = grad[v][a] * sc;
-                            if (clip[v]) rec.clip(v, sc);
+                            dp[v] = dot<D>(grad[v], offset[u]);
+                            const double at = Wi[v] + dp[v];
+                            const bool up = dp[v] > 0 && at > s.hi[v], down = dp[v] < 0 && at < s.lo[v];
+                            clip[v] = use && (up || down);
+                            bound[v] = dp[v] > 0 ? s.hi[v] : s.lo[v];
+                            any = any || clip[v];
                         }
-                    }
-                } else {  // reduced precision (:558-562): the offset, the face's change and the range relative to W_i in G
-                    if (!use) continue;
-                    G rg[D];
+                        if (use) rec.face(offset[u]);
+                        if (__any(any)) {
 #pragma unroll
-                    for (int a = 0; a < D; ++a) rg[a] = (G)offset[u][a];
+                            for (int v = 0; v < V; ++v) {
+                                // (bound - W) / dp where the bound is on the change's side of W, else 0
+                                const double q = Op::quotient(bound[v] - Wi[v], Op::by(dp[v]));
+                                const double sc = clip[v] ? (q > 0 ? q : 0.0) : 1.0;
 #pragma unroll
-                    for (int v = 0; v < V; ++v) {
-                        const G dp = dot<D>(grad[v], rg);
-                        if (dp > 0 && dp > s.hi[v]) {
-                            const G sc = s.hi[v] > 0 ? s.hi[v] / dp : G(0);
+                                for (int a = 0; a < D; ++a) grad[v][a] = grad[v][a] * sc;
+                                if (clip[v]) rec.clip(v, sc);
+                            }
+                        }
+                    } else {  // reduced precision (:558-562): the offset, the face's change and the range relative to W_i in G
+                        if (!use) continue;
+                        G rg[D];
 #pragma unroll
-                            for (int a = 0; a < D; ++a) grad[v][a] = grad[v][a] * sc;
-                        } else if (dp < 0 && dp < s.lo[v]) {
-                            const G sc = s.lo[v] < 0 ? s.lo[v] / dp : G(0);
+                        for (int a = 0; a < D; ++a) rg[a] = (G)offset[u][a];
 #pragma unroll
-                            for (int a = 0; a < D; ++a) grad[v][a] = grad[v][a] * sc;
+                        for (int v = 0; v < V; ++v) {
+                            const G dp = dot<D>(grad[v], rg);
+                            if (dp > 0 && dp > s.hi[v]) {
+                                const G sc = s.hi[v] > 0 ? s.hi[v] / dp : G(0);
+#pragma unroll
+                                for (int a = 0; a < D; ++a) grad[v][a] = grad[v][a] * sc;
+                            } else if (dp < 0 && dp < s.lo[v]) {
+                                const G sc = s.lo[v] < 0 ? s.lo[v] / dp : G(0);
+#pragma unroll
+                                for (int a = 0; a < D; ++a) grad[v][a] = grad[v][a] * sc;
+                            }
                         }
                     }
                 }
             }
-        }
-    }
-    if constexpr (Fast) {
-        if (!__all(ok || !here)) return false;
+        };
+        if (!exact || fast)
+            limit(std::true_type{});
+        else
+            limit(std::false_type{});
     }
     if (!here) {
         smallest = INFINITY;
-        return true;
+        return;
     }
     if constexpr (Moving) {
 #pragma unroll
@@ -619,18 +650,16 @@ __device__ __forceinline__ bool sweep_slice(const Geo& g, const Rows& r, double 
             }
         }
     }
-    return true;
 }
 
 template <int D, bool Moving, bool Grad, int Limit, int Rule, int Prec = 0>
-__global__ __launch_bounds__(CELL_BLOCK, Limit == 2 ? 1 : LUNA_SWEEP_WAVES) void k_sweep(Geo g, Rows r, Gas gas, double courant, Counters c) {
+__global__ __launch_bounds__(CELL_BLOCK, Limit == 2 ? 1 : Prec ? 3 : LUNA_SWEEP_WAVES) void k_sweep(Geo g, Rows r, Gas gas, double courant, Counters c) {
     reset_counters(c);
     __shared__ double rows[Stage<D>::DOUBLES];
     lds_double* lds = (lds_double*)rows;
     const int block = xcd_block();
     double smallest = INFINITY;
-    if (!sweep_slice<D, Moving, Grad, Limit, Rule, Prec, true>(g, r, courant, block, lds, smallest))
-        sweep_slice<D, Moving, Grad, Limit, Rule, Prec, false>(g, r, courant, block, lds, smallest);
+    sweep_slice<D, Moving, Grad, Limit, Rule, Prec>(g, r, courant, block, lds, smallest);
     block_min<CELL_BLOCK>(smallest, c.dt + (blockIdx.x % DT_SLOTS) * DT_STRIDE);
 }
 
@@ -685,7 +714,7 @@ __global__ __launch_bounds__(CELL_BLOCK, LUNA_LANE_WAVES(L)) void k_sweep_lanes(
             load_near<D>(g, base + t * SLICE, g.other[base + t * SLICE], n);
             surface += n.mag;
             smallest_face = fmin(smallest_face, n.mag);
-            s.add(g, n, xi, centroid, Wi, ci, ri, courant, 0.0);
+            s.template add<false>(g, n, xi, centroid, Wi, ci, ri, courant, 0.0);
         }
         surface = lanes_sum<L>(surface);
         smallest_face = lanes_min<L>(smallest_face);
