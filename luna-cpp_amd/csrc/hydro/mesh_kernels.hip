@@ -315,8 +315,8 @@ struct Sums {
         if constexpr (Moving) {
             if constexpr (Fast) operands.large(magnitude);
             if constexpr (Fast && D == 3) {  // face_angle<3>: 1 / pi rounded to nearest, as divisor() would give it
-                operands.small(magnitude);
-                const double angle = root(over(magnitude, Divisor{M_PI, M_1_PI}));
+                operands.small_or_zero(magnitude);
+                const double angle = root(over(magnitude, Divisor{M_PI, M_1_PI}));  // |A| = 0: a NaN, which the maximum passes by
                 max_angle = higher(max_angle, over(angle, Divisor{0.5 * dist, 2.0 * by_dist.y}));
             } else {
                 max_angle = fmax(max_angle, Op::quotient(face_angle<D>(magnitude), Divisor{0.5 * dist, 2.0 * by_dist.y}));
@@ -344,10 +344,10 @@ struct Sums {
             double dv[D];
 #pragma unroll
             for (int a = 0; a < D; ++a) dv[a] = n.W[1 + a] - Wi[1 + a];
-            // (a dv . d too small for the quotient's last bit is too small for vsig's, which is in range)
+            // (a dv . d too small for the quotient's last bit is too small for vsig's, which is in range or not positive)
             const double vsig = csi + n.cs - Op::quotient(dot<D>(dv, d), by_dist);
             if constexpr (Fast) {
-                operands.small(fabs(vsig));
+                operands.small_or_zero(vsig);
                 operands.large(vsig);
             }
             const double term = courant * Op::quotient(dist + ri, Op::by(vsig));
