@@ -154,7 +154,7 @@ struct luna_fv {
     Buf<double> q, grad, w, x, old_centroid, flux;
     Buf<unsigned int> exponents;  // grad16: the per-cell group exponents (int8 x 3)
     Buf<unsigned char> hll;       // the HLL fallback's per-cell compression flags
-    Buf<unsigned long long> counters;  // two sets of dt slots, then the fallbacks of the step's two flux passes
+    Buf<unsigned long long> counters;  // two sets of dt slots, then as many of the fallbacks of the step's two flux passes
     // the derivatives' rows (first use): luna::Derivs
     Buf<double> d_dq, d_dW, d_dgrad, d_dflux, d_sidebar, d_bbar, d_boundbar, d_out;
     Buf<int> d_extreme;
@@ -227,8 +227,7 @@ struct luna_fv {
     luna::Counters counters_now() const {
         return luna::Counters{counters.p + parity * luna::DT_WORDS, counters.p + (parity ^ 1) * luna::DT_WORDS, fallback_counters()};
     }
-    unsigned long long* fallback_counters() const { return counters.p + 2 * luna::DT_WORDS;
-    }
+    unsigned long long* fallback_counters() const { return counters.p + 2 * luna::DT_WORDS; }
 };
 
 namespace {
@@ -496,7 +495,7 @@ int flux_and_update(luna_fv* fv, int pass, double flux_dt, double apply_dt, doub
     const luna::Rows r = fv->rows();
     const luna::Gas gas = fv->gas();
     hipStream_t s = fv->stream;
-    unsigned long long* count = fv->fallback_counters() + (pass == 1 ? 1 : 0);
+    unsigned long long* count = fv->fallback_counters() + (pass == 1 ? luna::DT_WORDS : 0);
     const int riemann = fv->riemann(), order = fv->opt.order;
     if (prims) *prims = next_prims && fv->opt.update != LUNA_UPDATE_PER_CELL;
     if (fv->opt.update == LUNA_UPDATE_PER_CELL) {
@@ -576,7 +575,7 @@ int create(const luna_fv_options* opt, const luna_geometry* mesh, luna_fv** out,
     if ((e = fv->q.reserve(N * V)) != hipSuccess || (e = fv->count.reserve(N)) != hipSuccess ||
         (e = fv->grad.reserve(N * fv->grad_row())) != hipSuccess || (e = fv->w.reserve(N * D)) != hipSuccess ||
         (e = fv->cell.reserve(N * luna::CELL_ROW)) != hipSuccess || (e = fv->volume.reserve(N)) != hipSuccess ||
-        (e = fv->counters.reserve(2 * luna::DT_WORDS + 2)) != hipSuccess || (e = fv->geo_info.reserve(1)) != hipSuccess ||
+        (e = fv->counters.reserve(4 * luna::DT_WORDS)) != hipSuccess || (e = fv->geo_info.reserve(1)) != hipSuccess ||
         (e = fv->geo_flags.reserve(1)) != hipSuccess)
         return cleanup(fail(LUNA_ERR_MEMORY, std::string("luna: device allocation: ") + hipGetErrorString(e)));
     if (opt->limiter == LUNA_LIMITER_LEARNED) {
@@ -593,10 +592,10 @@ int create(const luna_fv_options* opt, const luna_geometry* mesh, luna_fv** out,
             (e = fv->steps.reserve(N * D)) != hipSuccess)
             return cleanup(fail(LUNA_ERR_MEMORY, std::string("luna: device allocation: ") + hipGetErrorString(e)));
     }
-    if (hipHostMalloc(reinterpret_cast<void**>(&fv->host), (8 + luna::DT_WORDS) * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess)
+    if (hipHostMalloc(reinterpret_cast<void**>(&fv->host), (8 + 2 * luna::DT_WORDS) * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess)
         return cleanup(fail(LUNA_ERR_MEMORY, "luna: pinned host allocation failed"));
-    std::vector<unsigned long long> init(2 * luna::DT_WORDS + 2, luna::INF_BITS);
-    init[2 * luna::DT_WORDS] = init[2 * luna::DT_WORDS + 1] = 0;
+    std::vector<unsigned long long> init(4 * luna::DT_WORDS, luna::INF_BITS);
+    std::fill(init.begin() + 2 * luna::DT_WORDS, init.end(), 0);
     if (hipMemcpy(fv->counters.p, init.data(), sizeof(unsigned long long) * init.size(), hipMemcpyHostToDevice) != hipSuccess)
         return cleanup(fail(LUNA_ERR_DEVICE, "luna: counter initialisation failed"));
     std::vector<double> zero(N * V, 0.0);
@@ -1246,10 +1245,13 @@ int luna_synchronize(void) {
 
 int luna_fv_fallbacks(luna_fv* fv, long long* count) {
     if (!fv || !count) return fail(LUNA_ERR_ARGUMENT, "luna_fv_fallbacks: null argument");
-    LUNA_HIP(hipMemcpyAsync(fv->host + 2, fv->fallback_counters(), 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, fv->stream));
+    unsigned long long* slots = fv->host + 8;
+    LUNA_HIP(hipMemcpyAsync(slots, fv->fallback_counters(), sizeof(unsigned long long) * 2 * luna::DT_WORDS, hipMemcpyDeviceToHost, fv->stream));
     LUNA_HIP(hipStreamSynchronize(fv->stream));
     LUNA_HIP(fv->prof.collect());
-    *count = static_cast<long long>(fv->host[2] + fv->host[3]);
+    unsigned long long sum = 0;
+    for (int k = 0; k < 2 * luna::DT_SLOTS; ++k) sum += slots[k * luna::DT_STRIDE];
+    *count = static_cast<long long>(sum);
     return LUNA_OK;
 }
 

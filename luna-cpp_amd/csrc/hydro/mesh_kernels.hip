@@ -77,11 +77,13 @@ __device__ __forceinline__ void block_min(double v, unsigned long long* out) {
         if (m < INFINITY) atomicMin(out, (unsigned long long)__double_as_longlong(m));
     }
 }
-// The first block resets the other dt slots and the step's fallback counters.
+// The first block resets the other dt slots and the step's fallback counts.
 __device__ __forceinline__ void reset_counters(const Counters& c) {
     if (blockIdx.x != 0) return;
-    if (threadIdx.x < DT_SLOTS) c.dt_next[threadIdx.x * DT_STRIDE] = INF_BITS;
-    if (threadIdx.x < 2) c.fallbacks[threadIdx.x] = 0;
+    if (threadIdx.x < DT_SLOTS) {
+        c.dt_next[threadIdx.x * DT_STRIDE] = INF_BITS;
+        c.fallbacks[threadIdx.x * DT_STRIDE] = c.fallbacks[DT_WORDS + threadIdx.x * DT_STRIDE] = 0;
+    }
 }
 template <int B>
 __device__ __forceinline__ void block_count(int v, unsigned long long* out) {
@@ -93,7 +95,7 @@ __device__ __forceinline__ void block_count(int v, unsigned long long* out) {
     if (threadIdx.x == 0) {
         int s = 0;
         for (int k = 0; k < (int)(blockDim.x >> 6); ++k) s += part[k];
-        if (s) atomicAdd(out, (unsigned long long)s);
+        if (s) atomicAdd(out + (blockIdx.x % DT_SLOTS) * DT_STRIDE, (unsigned long long)s);
     }
 }
 
