@@ -186,7 +186,7 @@ struct luna_fv {
     bool mesh_ok = false;  // the last mesh given was accepted
     bool far_offsets = false;
     // The accepted mesh's arrays: the step reads its face arrays in place (a device mesh's, or the copies of a host mesh in
-    // the src_ buffers); `records` once the derivatives' face records are built for it.
+    // the src_ buffers); `records` once its face records are built.
     luna::MeshIn mesh{};
     bool records = false;
 
@@ -250,9 +250,7 @@ int check_geometry(const luna_geometry* m, int D, int N) {
 // the steps that follow, until the next mesh; the cell arrays and lists are not read after this returns. A malformed
 // mesh (CSR offsets, cell or face indices out of range, more than 2^31 slots) is refused, and the handle takes no step
 // until a valid mesh is set.
-int records(luna_fv* fv);
-
-int derive(luna_fv* fv, const luna_geometry* m, luna::MeshIn in, bool eager_records) {
+int derive(luna_fv* fv, const luna_geometry* m, luna::MeshIn in) {
     const int D = fv->D, N = fv->N;
     fv->mesh_ok = false;
     if (fv->opt.motion == LUNA_MOTION_MOVING) {
@@ -268,7 +266,6 @@ int derive(luna_fv* fv, const luna_geometry* m, luna::MeshIn in, bool eager_reco
     }
     hipStream_t s = fv->stream;
     LUNA_HIP(fv->slice.reserve(S));
-    LUNA_HIP(fv->facerec.reserve(static_cast<size_t>(F) * luna::FACE_ROW));
     LUNA_HIP(fv->flux.reserve(static_cast<size_t>(F) * fv->V));
     LUNA_HIP(hipMemsetAsync(fv->geo_flags.p, 0, sizeof(unsigned int), s));
     LUNA_HIP(timed(fv->prof, s, "geometry_cells", [&] {
@@ -310,8 +307,6 @@ int derive(luna_fv* fv, const luna_geometry* m, luna::MeshIn in, bool eager_reco
     fv->mesh.centroid = fv->mesh.volume = fv->mesh.positions = nullptr;
     fv->records = false;
     fv->mesh_ok = true;
-    if (eager_records)
-        if (int rc = records(fv)) return rc;
     for (int a = 0; a < 3; ++a) fv->side[a] = a < D ? m->side[a] : 0.0;
     fv->grid.step = m->step;
     fv->grid.per_step = m->step > 0 ? 1.0 / m->step : 0.0;
@@ -338,7 +333,7 @@ luna::MeshIn mesh_in(const luna_geometry* m) {
 // A mesh in device memory (the arrays the producer left on the GPU), read in place.
 int upload_device(luna_fv* fv, const luna_geometry* m) {
     if (int rc = check_geometry(m, fv->D, fv->N)) return rc;
-    return derive(fv, m, mesh_in(m), false);
+    return derive(fv, m, mesh_in(m));
 }
 
 // A mesh in host memory: its arrays are copied to the handle's device buffers, then derived as a device mesh. Host
@@ -378,14 +373,16 @@ int upload(luna_fv* fv, const luna_geometry* m) {
     in.centroid = centroid;
     in.volume = volume;
     in.positions = positions;
-    return derive(fv, m, in, true);
+    return derive(fv, m, in);
 }
 
-// The derivatives read each face as one 64 B record (k_geo_faces, from the face arrays the step reads in place; the pass
-// has checked their cell indices). Built on their first use of a mesh, stream-ordered; a host mesh's at once.
+// The moving step's derivatives and the per-cell update read each face as one 64 B record (k_geo_faces, from the face arrays
+// the step reads in place; the pass has checked their cell indices). Built on their first use of a mesh, stream-ordered, before
+// the geo() that their kernels take: it holds the records' address.
 int records(luna_fv* fv) {
     if (fv->records || !fv->mesh_ok) return LUNA_OK;
     hipStream_t s = fv->stream;
+    LUNA_HIP(fv->facerec.reserve(static_cast<size_t>(fv->F) * luna::FACE_ROW));
     LUNA_HIP(timed(fv->prof, s, "geometry_faces", [&] {
         return fv->D == 3 ? luna::launch_geometry_faces<3>(s, fv->mesh, fv->facerec.p, fv->geo_flags.p)
                           : luna::launch_geometry_faces<2>(s, fv->mesh, fv->facerec.p, fv->geo_flags.p);
@@ -491,6 +488,8 @@ int ensure_swept(luna_fv* fv) {
 // with next_prims), else the next time_step computes them.
 int flux_and_update(luna_fv* fv, int pass, double flux_dt, double apply_dt, double unit, bool next_prims, bool* prims = nullptr) {
     const luna::Grid* drift = pass == 0 ? &fv->grid : nullptr;
+    if (fv->opt.update == LUNA_UPDATE_PER_CELL)  // the per-cell loop reads each face's record
+        if (int rc = records(fv)) return rc;
     const luna::Geo g = fv->geo();
     const luna::Rows r = fv->rows();
     const luna::Gas gas = fv->gas();
@@ -499,7 +498,6 @@ int flux_and_update(luna_fv* fv, int pass, double flux_dt, double apply_dt, doub
     const int riemann = fv->riemann(), order = fv->opt.order;
     if (prims) *prims = next_prims && fv->opt.update != LUNA_UPDATE_PER_CELL;
     if (fv->opt.update == LUNA_UPDATE_PER_CELL) {
-        if (int rc = records(fv)) return rc;  // the per-cell loop reads each face's record
         LUNA_HIP(timed(fv->prof, s, pass < 0 || pass == 2 ? "fluxes_and_update" : pass == 0 ? "fluxes_and_update_pass1" : "fluxes_and_update_pass2", [&] {
             return fv->D == 3 ? luna::launch_fluxes_and_update<3>(s, g, r, gas, riemann, order, pass, flux_dt, apply_dt, unit, drift, count)
                               : luna::launch_fluxes_and_update<2>(s, g, r, gas, riemann, order, pass, flux_dt, apply_dt, unit, drift, count);
@@ -716,7 +714,6 @@ int derivatives_ready(luna_fv* fv, const char* what) {
     if (fv->opt.sweep_lanes > 1) return fail(LUNA_ERR_LOGIC, std::string(what) + ": derivatives of the one-lane sweep");
     if (fv->begun) return fail(LUNA_ERR_LOGIC, std::string(what) + ": a moving step is between begin and finish");
     if (!fv->mesh_ok) return fail(LUNA_ERR_LOGIC, "luna: the last mesh given was refused; set a valid mesh first");
-    if (int rc = records(fv)) return rc;
     const size_t N = fv->N, V = fv->V, F = fv->F;
     LUNA_HIP(fv->d_dq.reserve(N * V));
     LUNA_HIP(fv->d_dW.reserve(N * V));
@@ -885,7 +882,6 @@ int luna_fv_step_adjoint_noalloc(luna_fv* fv, double dt, double* qbar) {
                                            std::to_string(SCRATCH_BYTES) + " of the library's scratch (use luna_fv_step_adjoint)");
     w.dq = qbar;  // read only: the cotangent after the step
     hipStream_t s = fv->stream;
-    if (int rc = records(fv)) return rc;  // launches only: the records' memory is the handle's, reserved with the mesh
     if (int rc = primitives(fv)) return rc;  // the forward's rows at Q: primitives and the limited gradients
     if (int rc = sweep(fv, 1.0)) return rc;
     const luna::Geo g = fv->geo();
@@ -922,6 +918,7 @@ int luna_fv_moving_adjoint(luna_fv* fv, double dt, const luna_geometry* mesh0, c
     const int row_width = D == 3 ? 2 * (5 + 15 + 3) + 9 : 2 * (4 + 8 + 2) + 6;
     // t^n: its mesh and positions, W, the limited gradients and point velocities (the sweep keeps c^n), the grid steps.
     if (int rc = luna_fv_set_geometry(fv, mesh0)) return rc;  // and x^n
+    if (int rc = fv->opt.order == 0 ? records(fv) : LUNA_OK) return rc;  // at order 1 the passes come after the uploads below
     if (int rc = primitives(fv)) return rc;
     if (int rc = sweep(fv, 1.0)) return rc;
     if (fv->opt.order == 1) {
@@ -992,6 +989,7 @@ int luna_fv_moving_adjoint(luna_fv* fv, double dt, const luna_geometry* mesh0, c
     // Pass 2 on t^n+1 (the rows W^n, g^n, c^n and the steps stay), then x^n+1's bar with its geometry's adjoint.
     fv->begun = true;  // keeps W, g across the upload
     int rc = upload(fv, mesh1);
+    if (rc == LUNA_OK) rc = records(fv);
     fv->begun = false;
     if (rc != LUNA_OK) return rc;
     {
@@ -1013,6 +1011,7 @@ int luna_fv_moving_adjoint(luna_fv* fv, double dt, const luna_geometry* mesh0, c
     // Back to t^n: x^n's bar starts as x^n+1's (x^n+1 = x^n + dt w-hat), w-hat's gets dt of it unless the steps are held.
     fv->begun = true;
     rc = upload(fv, mesh0);
+    if (rc == LUNA_OK) rc = records(fv);
     fv->begun = false;
     if (rc != LUNA_OK) return rc;
     LUNA_HIP(hipMemcpyAsync(fv->m_xbar.p, hx.data(), sizeof(double) * ND, hipMemcpyHostToDevice, s));
@@ -1062,6 +1061,7 @@ int luna_fv_moving_tangent(luna_fv* fv, double dt, const luna_geometry* mesh0, c
     const bool limit = fv->opt.limiter == LUNA_LIMITER_FACE_CENTROID, order0 = fv->opt.order == 0;
     // t^n: its mesh and positions, W, the limited gradients and point velocities, c^n and the grid steps
     if (int rc = luna_fv_set_geometry(fv, mesh0)) return rc;
+    if (int rc = records(fv)) return rc;
     if (int rc = primitives(fv)) return rc;
     if (int rc = sweep(fv, 1.0)) return rc;
     if (!order0) {
@@ -1119,6 +1119,7 @@ int luna_fv_moving_tangent(luna_fv* fv, double dt, const luna_geometry* mesh0, c
         LUNA_HIP(hipMemcpyAsync(fv->t_dxf.p, hxf.data(), sizeof(double) * F1 * D, hipMemcpyHostToDevice, s));
         fv->begun = true;  // keeps W, g across the upload
         int rc = upload(fv, mesh1);
+        if (rc == LUNA_OK) rc = records(fv);
         fv->begun = false;
         if (rc != LUNA_OK) return rc;
         t.dx = fv->t_dx1.p;

@@ -44,7 +44,7 @@ struct Geo {
     const int* other;   // slots: the cell on the other side of the entry's face
     double* cell;       // N x CELL_ROW (the kernels write only the primitive half)
     const double* volume;  // N: the cell rows' volumes again, densely, for the kernels that read no other geometry
-    const double* face; // F x FACE_ROW records, for the derivatives (built on their first use of a mesh)
+    const double* face; // F x FACE_ROW records, for the moving step's derivatives and the per-cell update (built on their first use of a mesh)
     // The mesh's face arrays, read in place as the reference reads the mesh's views (finite_volume.hpp:257-327): owner
     // and neighbour (F), area vectors and face centroids relative to the owner's generator (F x D)
     const int* owner;
@@ -122,7 +122,8 @@ struct Grid {
 // smallest the host takes: atomics to one address are served one after the other, about 11 ns each on MI355X, so that the
 // 4096 wavefronts of a 511^2 sweep took 76 us with one address and take 38 with 32. (A line's kernels use the first alone,
 // but for the static step of a long line.) The fallback counts of a flux pass are spread the same way, for a flow with
-// fallbacks in most wavefronts: a flux of 64^3 cells with 2.3 million took 393 us with one address and takes 93 with 32, against 89 with none.
+// fallbacks in most wavefronts: a flux of 64^3 cells with 2.3 million took 393 us with one address and takes 93 with 32, against
+// 89 with none.
 constexpr int DT_SLOTS = 32, DT_STRIDE = 16, DT_WORDS = DT_SLOTS * DT_STRIDE;
 struct Counters {
     unsigned long long* dt;         // the min-reduction this sweep writes
@@ -159,7 +160,8 @@ hipError_t launch_drift(hipStream_t s, const Geo& g, const Rows& r, double dt);
 // The geometry pass (geometry_kernels.hip), in this order on one stream: cells (the geometry half of the cell rows, the
 // list lengths, each slice's longest list into slice), scan (slice's first slots, the total into info[0]), pairs (the
 // faces' owner and neighbour checked); the host then checks the flags and sizes the slot arrays; slots (lists, other
-// cells, |A| and face offsets). faces (the F x FACE_ROW records) runs on a derivative's first use of a mesh.
+// cells, |A| and face offsets). faces (the F x FACE_ROW records) runs on the first use of a
+// mesh by the moving step's derivatives or the per-cell update.
 template <int D>
 hipError_t launch_geometry_cells(hipStream_t s, const MeshIn& m, double* cell, double* volume, int* count, int* slice, unsigned int* flags);
 hipError_t launch_geometry_scan(hipStream_t s, int* slice, int S, long long* info, unsigned int* flags);

@@ -210,3 +210,39 @@ def test_derivatives_on_a_device_mesh_equal_the_host_meshs():
     finally:
         dev.close()
         host.close()
+
+
+def test_face_records_are_built_for_what_reads_them():
+    """The 64 B face records: built once for a mesh by the per-cell update and by the moving step's derivatives, never by the
+    static derivatives, which read the face arrays and the slots; host and device meshes alike."""
+    m = cases.voronoi(7, 3)
+    q = cases.rough_state(m)
+    rng = np.random.default_rng(5)
+    dq = rng.standard_normal(np.shape(q))
+
+    def built(fv):
+        return fv.kernel_times().get("geometry_faces", (0, 0))[0]
+
+    for given in (m, hydro.DeviceMesh(m)):
+        fv = hydro.FiniteVolume(given, GAMMA)
+        cell = hydro.FiniteVolume(given, GAMMA, update="per_cell")
+        try:
+            fv.profile(True)
+            fv.set_geometry(given)
+            fv.set_state(q)
+            dt = fv.time_step(0.3)
+            fv.step_adjoint(dt, dq)
+            fv.step_tangent(dt, dq)
+            fv.step(dt)
+            fv.state()
+            assert built(fv) == 0
+            cell.profile(True)
+            cell.set_geometry(given)
+            cell.set_state(q)
+            cell.step(dt)
+            cell.step(dt)
+            cell.state()
+            assert built(cell) == 1
+        finally:
+            fv.close()
+            cell.close()
