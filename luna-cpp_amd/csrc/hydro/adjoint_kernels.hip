@@ -383,8 +383,8 @@ __global__ __launch_bounds__(BLOCK) void k_flux_tangent(Geo g, Rows r, Gas gas, 
     constexpr int V = D + 2;
     using Staged = StagedSide<D, 0>;
     constexpr int GRAD = Staged::GRAD;
-    __shared__ double rows[Staged::DOUBLES + 64 * 2 * GRAD];
-    lds_double* lds = (lds_double*)rows;
+    __shared__ StagedRows<Staged::DOUBLES + 64 * 2 * GRAD> rows;
+    lds_double* lds = rows.lds();
     lds_double* tangents = lds + Staged::DOUBLES;
     const int lane = threadIdx.x, f = blockIdx.x * BLOCK + lane, at = min(f, g.F - 1);
     const int j = g.neighbour[at];
@@ -486,8 +486,8 @@ template <int D>
 __global__ __launch_bounds__(BLOCK) void k_face_adjoint(Geo g, Rows r, Gas gas, int riemann, double dt, const double* qbar, double* sidebar) {
     constexpr int V = D + 2;
     using Staged = StagedSide<D, 0>;
-    __shared__ double rows[Staged::DOUBLES];
-    lds_double* lds = (lds_double*)rows;
+    __shared__ StagedRows<Staged::DOUBLES> rows;
+    lds_double* lds = rows.lds();
     const int lane = threadIdx.x, f = blockIdx.x * BLOCK + lane, at = min(f, g.F - 1);
     Staged::fetch(g, r, g.neighbour[at], true, lds, lane);
     FaceIn<D> face;

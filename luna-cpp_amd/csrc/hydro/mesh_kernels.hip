@@ -657,8 +657,8 @@ __device__ __forceinline__ void sweep_slice(const Geo& g, const Rows& r, double 
 template <int D, bool Moving, bool Grad, int Limit, int Rule, int Prec = 0>
 __global__ __launch_bounds__(CELL_BLOCK, Limit == 2 ? 1 : Prec ? 3 : LUNA_SWEEP_WAVES) void k_sweep(Geo g, Rows r, Gas gas, double courant, Counters c) {
     reset_counters(c);
-    __shared__ double rows[Stage<D>::DOUBLES];
-    lds_double* lds = (lds_double*)rows;
+    __shared__ StagedRows<Stage<D>::DOUBLES> rows;
+    lds_double* lds = rows.lds();
     const int block = xcd_block();
     double smallest = INFINITY;
     sweep_slice<D, Moving, Grad, Limit, Rule, Prec>(g, r, courant, block, lds, smallest);
@@ -1071,8 +1071,8 @@ template <int D, int Pass, int Riemann, int Prec = 0>
 __global__ __launch_bounds__(CELL_BLOCK, LUNA_FLUX_WAVES) void k_flux(Geo g, Rows r, Gas gas, int order, double dt, double unit, unsigned long long* fallbacks) {
     constexpr int V = D + 2;
     using Staged = StagedSide<D, Prec>;
-    __shared__ double rows[Staged::DOUBLES];
-    lds_double* lds = (lds_double*)rows;
+    __shared__ StagedRows<Staged::DOUBLES> rows;
+    lds_double* lds = rows.lds();
     const int lane = threadIdx.x, f = xcd_block() * CELL_BLOCK + lane;
     int count = 0;
     if (g.F > 0) {

@@ -21,6 +21,17 @@ struct Near {
 typedef __attribute__((address_space(3))) double lds_double;
 typedef double double2v __attribute__((ext_vector_type(2)));
 
+// A work-group's staged rows in LDS. They are filled and read 16 B at a time, which a plain array of doubles does not promise
+// the alignment of (another __shared__ variable before it may leave it at 8).
+template <int DOUBLES>
+struct alignas(16) StagedRows {
+    double at[DOUBLES];
+    static_assert(DOUBLES % 2 == 0, "whole 16 B chunks");
+
+    __device__ __forceinline__ lds_double* lds() { return (lds_double*)at; }
+};
+static_assert(alignof(StagedRows<2>) == sizeof(double2v), "ds_read_b128 and the 16 B loads to LDS");
+
 // A wavefront's neighbour rows through LDS. A lane that loads its own neighbour's row itself touches a 128 B line per 16 B
 // load, and a CU's L1 looks up one line a cycle: the rows of 64 neighbours cost 7 x 64 lookups, which bound the list walk
 // (5.6 thousand cycles an entry at 12 wavefronts a CU). Here the 16 B chunks of all 64 rows are dealt to the lanes in order
