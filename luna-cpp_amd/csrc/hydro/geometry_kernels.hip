@@ -164,7 +164,7 @@ __global__ __launch_bounds__(BLOCK) void k_geo_pairs(MeshIn m, unsigned int* fla
 // take consecutive entries (so the list and the faces a cell owns, numbered consecutively, are read in runs); each finds
 // its cell among the 16 offsets and computes its slot's values into LDS, laid out as the slots are; then the work-group
 // writes each (entry t, array) as one whole run of 16 slots (one 128-byte line for the doubles). Padding slots (t at or
-// past the cell's list length) get zeros. A quarter deeper than QUARTER_DEPTH entries writes the rest straight to memory.
+// past the cell's list length) get zeros: the sweep reads them and leaves them out. A quarter deeper than QUARTER_DEPTH entries writes the rest straight to memory.
 // The CSR offsets were checked by k_geo_cells (the host runs this only when they passed).
 // What bounds it is the latency of an entry's chain (list, cells, face arrays), so the wavefronts in flight: 32 entries deep
 // (20 KiB of LDS, 8 work-groups a CU) takes 0.46 ms at 104^3, 48 deep (5 a CU) 0.51; before, with the cells' own positions and
@@ -287,6 +287,8 @@ __global__ __launch_bounds__(SLOT_BLOCK) void k_geo_slots(MeshIn m, const int* _
         const long long sl = base + (long long)t * SLICE + quarter * QUARTER + l;
         list[sl] = 0;
         other[sl] = 0;
+#pragma unroll
+        for (int a = 0; a <= D; ++a) slot[a * slots + sl] = 0.0;
     }
     if (bad) flag(flags, bad);
 }

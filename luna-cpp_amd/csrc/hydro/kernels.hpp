@@ -31,8 +31,8 @@ struct FaceAt {
 };
 
 // Face lists in slices of 64 cells (one wavefront): entry t of cell i sits in slot slice[i / 64] + 64 t + i % 64, so the
-// t-th entries of a wavefront's cells are one contiguous run; a slice is as long as its longest list (the rest is padding
-// that no kernel reads). Within a cell the entries keep the mesh's list order.
+// t-th entries of a wavefront's cells are one contiguous run; a slice is as long as its longest list (the rest is padding:
+// zeros, which name cell 0; the sweep reads it and leaves it out). Within a cell the entries keep the mesh's list order.
 constexpr int SLICE = 64;
 
 // The mesh as the kernels read it (device pointers): finite_volume.hpp:257-327 Geometry, packed.
