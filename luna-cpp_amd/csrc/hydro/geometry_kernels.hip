@@ -22,14 +22,6 @@ namespace {
 
 constexpr int BLOCK = 256;
 
-// The logical block of this work-group: work-groups go to the 8 XCDs in turn (block b to XCD b mod 8), so XCD x takes a
-// contiguous run, and the faces that neighbouring cells share are fetched into one L2.
-__device__ __forceinline__ int xcd_block() {
-    const int b = blockIdx.x, n = gridDim.x;
-    const int q = n >> 3, rem = n & 7, x = b & 7, k = b >> 3;
-    return x * q + min(x, rem) + k;
-}
-
 __device__ __forceinline__ void flag(unsigned int* flags, unsigned int bit) { atomicOr(flags, bit); }
 
 template <int D>

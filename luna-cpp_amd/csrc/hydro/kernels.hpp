@@ -131,6 +131,15 @@ struct Counters {
     unsigned long long* fallbacks;  // 2 x DT_WORDS: face sides that took the cell's state, per flux pass of the step
 };
 
+// The logical block of this work-group. Work-groups go to the 8 XCDs in turn (block b to XCD b mod 8), so XCD x gets the
+// contiguous logical run [x q + min(x, r), ...) of q + (x < r) blocks (q = n / 8, r = n mod 8), a bijection: the rows that
+// neighbouring cells and faces share are fetched into one L2.
+__device__ __forceinline__ int xcd_block() {
+    const int b = blockIdx.x, n = gridDim.x;
+    const int q = n >> 3, rem = n & 7, x = b & 7, k = b >> 3;
+    return x * q + min(x, rem) + k;
+}
+
 // Kernel launchers (api.hip calls these; each returns the HIP launch status).
 template <int D>
 hipError_t launch_primitives(hipStream_t s, const Geo& g, const Rows& r, const Gas& gas);

@@ -43,14 +43,6 @@ namespace {
 // early frees its slot without waiting for the others of its group; the rest run 256.
 constexpr int BLOCK = 256, CELL_BLOCK = 64;
 
-// The logical block of this work-group. Work-groups go to the 8 XCDs in turn (block b to XCD b mod 8), so XCD x gets the
-// contiguous logical run [x q + min(x, r), ...) of q + (x < r) blocks (q = n / 8, r = n mod 8): a bijection.
-__device__ __forceinline__ int xcd_block() {
-    const int b = blockIdx.x, n = gridDim.x;
-    const int q = n >> 3, rem = n & 7, x = b & 7, k = b >> 3;
-    return x * q + min(x, rem) + k;
-}
-
 __device__ __forceinline__ double wave_min(double v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o));
