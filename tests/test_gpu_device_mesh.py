@@ -190,8 +190,8 @@ def test_release_mesh_copies_a_device_meshs_face_arrays():
 
 
 def test_derivatives_on_a_device_mesh_equal_the_host_meshs():
-    """On a device mesh the derivatives' face records are built on their first use (from the face arrays read in place):
-    the tangent and the adjoint equal those of the same mesh given as host arrays, to the bit."""
+    """On a device mesh the derivatives read the producer's face arrays in place: the tangent and the adjoint equal those of
+    the same mesh given as host arrays, to the bit."""
     say("derivatives on a device mesh")
     m = cases.voronoi(8, 3)
     q = cases.rough_state(m)

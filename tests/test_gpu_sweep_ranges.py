@@ -1,6 +1,7 @@
 """The sweep at the ends of its ranges against the oracle, to the bit: cell counts around a wavefront's 64, meshes with many
-tiny faces (left out of the limiter's range), and operands outside the exponents that its fast divisions and square roots
-take (boxes of 2^-255 and velocities of 2^-950 take the general operators; boxes of 2^-130 and 2^60 are still inside).
+tiny faces (left out of the limiter's range) or faces of area zero, and operands outside the exponents that its fast
+divisions and square roots take (boxes of 2^-255 take the general operators, velocities of 2^-950 do for their own systems and
+clips; boxes of 2^-130 and 2^60 are still inside), with the derivatives' fit beside it; and that the latter cost little.
 """
 import numpy as np
 import pytest
