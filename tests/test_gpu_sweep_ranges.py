@@ -172,3 +172,15 @@ def test_faces_of_area_zero_do_not_cost_a_second_walk():
     ratio = sweep_ms(without_extent(m, 150), q, motion="moving") / sweep_ms(m, q, motion="moving")
     print("|A| = 0: %.2f of the time" % ratio, flush=True)
     assert ratio < 1.45
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("limiter", ["face", "none"])
+@pytest.mark.parametrize("power", [-249, -240, -225, 110, 130, 240])
+def test_box_scales_between_the_ranges(dim, limiter, power):
+    """Boxes in which one part only is out of the fast operators' range: the Cholesky factor's diagonal (2^-225 and below, 2^130
+    and above), the right-hand sides, the face offsets (2^110 and above), while the separations are still inside."""
+    base = cases.voronoi(10 if dim == 3 else 24, dim)
+    m = scaled(base, 2.0 ** power)
+    q = cases.rough_state(base) / base["volume"][:, None] * m["volume"][:, None]
+    compare(m, q, limiter=limiter)
